@@ -6,9 +6,8 @@
 //     ops.go:788-807 -> bf16_matmul.go:159-173): the MFMA weight-streaming
 //     kernel in gemv.hip;
 //   - every other transpose/dtype combination, and every batch of more than
-//     one entry: k_matmul_mfma, one launch over the batch, each operand
-//     gathered through its own layout and dtype into bf16 matrix-core terms
-//     (not a hot path of the decode step).
+//     one entry: k_mm, one launch over the batch, a kernel per operand
+//     layout and dtype, each operand split into bf16 matrix-core terms.
 #include <algorithm>
 
 #include "common.h"
@@ -19,125 +18,371 @@ int launch_gemm_bf16w(hipStream_t s, const float* A, const uint16_t* W, const fl
                       const float* residual, const OutDesc& od, int M, int N, int K, int epilogue,
                       bool act_bf16);
 
-// C[b] = opA(A[b]) @ opB(B[b]) on the matrix cores for every transpose /
-// dtype combination of metal_mps_matmul_dt (one launch for the whole batch,
-// blockIdx.z = batch entry). Block tile 64 x 64, K stepped by 32; each
-// operand tile is gathered through its own layout into LDS as bf16 terms
-// in [row][k] order (NTA / NTB terms: 1 for a bf16 operand, 3 for an f32
-// one), then 4 waves (2 x 2, 32 x 32 each) run v_mfma_f32_16x16x32_bf16
-// over the term products whose term indices sum to at most 2 (the rest lie
-// below f32 rounding), accumulating in f32. Not a hot path of the decode
-// step: the gather is per element (bf16 storage is one exact term; f32 is
-// hi, the value truncated to bf16, mid, the remainder truncated to bf16, and
-// lo, what is left rounded to bf16: x = hi + mid + lo to ~2^-25 relative, so
-// f32 x f32 products carry f32-level error).
-constexpr int kMmBK = 32, kMmLD = kMmBK + 8;  // LDS row: 40 bf16 (80 bytes)
-
-template <int NTA, int NTB>
-__global__ __launch_bounds__(256) void k_matmul_mfma(const void* __restrict__ A, const void* __restrict__ B,
-                                                     float* __restrict__ C, int M, int N, int K, int transA,
-                                                     int transB) {
-    __shared__ __align__(16) uint16_t As[NTA][64][kMmLD];
-    __shared__ __align__(16) uint16_t Bs[NTB][64][kMmLD];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1, r = lane & 15, g = lane >> 4;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const size_t bA = (size_t)blockIdx.z * M * K, bB = (size_t)blockIdx.z * K * N;
-    floatx4 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // one raw buffer resource per operand over this batch entry (< 2 GiB,
-    // host check): elements outside the matrix get an out-of-range offset and
-    // read as zero, so all 16 of a thread's element loads go out together (a
-    // load under a bounds branch waits for the one before it)
-    constexpr int EA = NTA == 1 ? 2 : 4, EB = NTB == 1 ? 2 : 4;
-    static_assert(NTA == 1 || NTA == 3, "bf16: one term, f32: three");
-    static_assert(NTB == 1 || NTB == 3, "bf16: one term, f32: three");
-    const __amdgpu_buffer_rsrc_t ra = make_rsrc(reinterpret_cast<const char*>(A) + bA * EA, (long long)M * K * EA);
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(reinterpret_cast<const char*>(B) + bB * EB, (long long)K * N * EB);
-    auto ld = [](__amdgpu_buffer_rsrc_t rs, int off, bool half) -> uint32_t {
-        return half ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0)
-                    : __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0);
-    };
-    // the operand's terms: bf16 storage is exact; f32 v = hi + mid + lo (hi
-    // and mid truncations, each remainder exact in f32, lo rounded)
-    auto terms = [](uint32_t bits, bool half, uint16_t (&t)[3]) {
-        if (half) {
-            t[0] = (uint16_t)bits;
-            t[1] = t[2] = 0;
-            return;
-        }
-        const float v = __uint_as_float(bits);
-        const uint32_t u = bits & 0xffff0000u;
-        const float r1 = v - __uint_as_float(u);
-        const uint32_t u1 = __float_as_uint(r1) & 0xffff0000u;
-        t[0] = (uint16_t)(u >> 16);
-        t[1] = (uint16_t)(u1 >> 16);
-        t[2] = __builtin_bit_cast(uint16_t, (__bf16)(r1 - __uint_as_float(u1)));
-    };
-    for (int k0 = 0; k0 < K; k0 += kMmBK) {
-        // 64 x 32 elements per operand, 8 per thread: thread t takes row
-        // t / 4 (of the tile) and k 8 * (t % 4) .. +8, each element read
-        // through the operand's stored layout
-        const int row = tid >> 2, m = m0 + row, n = n0 + row;
-        uint32_t av[8], bv[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int k = k0 + 8 * (tid & 3) + e;
-            const int oa = (m < M && k < K) ? (transA ? k * M + m : m * K + k) * EA : kOutOfRange;
-            const int ob = (n < N && k < K) ? (transB ? n * K + k : k * N + n) * EB : kOutOfRange;
-            av[e] = ld(ra, oa, NTA == 1);
-            bv[e] = ld(rb, ob, NTB == 1);
-        }
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int kk = 8 * (tid & 3) + e;
-            uint16_t t[3];
-            terms(av[e], NTA == 1, t);
-#pragma unroll
-            for (int q = 0; q < NTA; q++) As[q][row][kk] = t[q];
-            terms(bv[e], NTB == 1, t);
-#pragma unroll
-            for (int q = 0; q < NTB; q++) Bs[q][row][kk] = t[q];
-        }
-        __syncthreads();
-        bf16x8 af[2][NTA], bfr[2][NTB];
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int t = 0; t < NTA; t++)
-                af[i][t] = *reinterpret_cast<const bf16x8*>(&As[t][wm * 32 + i * 16 + r][8 * g]);
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int t = 0; t < NTB; t++)
-                bfr[j][t] = *reinterpret_cast<const bf16x8*>(&Bs[t][wn * 32 + j * 16 + r][8 * g]);
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-#pragma unroll
-                for (int ta = 0; ta < NTA; ta++)
-#pragma unroll
-                    for (int tb = 0; tb < NTB; tb++)
-                        if (ta + tb <= 2) acc[i][j] = mfma16x16x32(af[i][ta], bfr[j][tb], acc[i][j]);
-        __syncthreads();
+// ---------------------------------------------------------------------------
+// k_mm: C[b] = opA(A[b]) @ opB(B[b]) on the matrix cores, one launch for the
+// whole batch (blockIdx.z = batch entry), a kernel per operand layout and
+// dtype.
+//
+// Terms: bf16 storage is one exact term; an f32 value is hi (truncated to
+// bf16), mid (the remainder truncated) and lo (what is left, rounded): x =
+// hi + mid + lo to ~2^-25 relative. The term products with ta + tb <= 2 are
+// kept (the rest lie below f32 rounding) and accumulated in f32 by
+// v_mfma_f32_16x16x32_bf16: one product for bf16 x bf16, three for f32 x
+// bf16, six for f32 x f32.
+//
+// A block takes a T x T tile of C (4 waves of T/2 x T/2) and steps K by BK.
+// Each thread loads a patch of each operand with the widest loads its layout
+// allows (8 k of P rows), splits it into terms once, and writes them to LDS
+// in [term][row][k] order, 16 bytes at a time, with the 16-byte chunks
+// XOR-swizzled so that neither the writes nor the 16-row fragment reads
+// conflict. The next step's loads are issued before a step's MFMAs: up to
+// 1024^3 the chain of K steps binds (load latency, split, LDS, MFMAs), above
+// it the matrix cores (f32 x f32 at 2000^3 runs them at 730 TFLOP/s). Rows
+// past the matrix are clamped into it (computed, never stored) and the loads
+// need only element alignment, so odd sizes run the same loop; only a last
+// step that is ragged in K, or whose row-contiguous loads would run past the
+// operand's end, is gathered element by element through a buffer resource
+// whose out-of-range reads are zeros.
+// The products are formed as (B fragment) x (A fragment), which leaves each
+// lane 4 consecutive columns of one row of C: one 16-byte store.
+// Tile sizes and what they measured: launch_mm.
+template <int T_, int BK_, bool F32>
+struct MmOperand {
+    static constexpr int T = T_, BK = BK_;
+    static constexpr int NT = F32 ? 3 : 1, E = F32 ? 4 : 2;
+    static constexpr int CH = BK / 8;           // 16-byte chunks per LDS row
+    static constexpr int P = T * BK / 8 / 256;  // rows per thread patch
+    static constexpr int ELEMS = NT * T * BK;   // LDS elements per stage
+    static_assert(P >= 1 && T % P == 0, "one patch per thread");
+    __device__ static __forceinline__ int swz(int row, int c) {
+        return CH == 8 ? (c ^ (row & 7)) : (c ^ ((row >> 1) & 3));
     }
-    // lane holds rows 4g..4g+3 of column r in each 16 x 16 fragment
-    float* Cb = C + (size_t)blockIdx.z * M * N;
+    // the 16-byte words of one patch: [row][8 k] of raw storage
+    struct Patch {
+        uint32_t w[P][8 * E / 4];
+    };
+    // k-contiguous patches: chunk tid + 256 i of the step (row q / CH, k 8 (q % CH));
+    // row-contiguous: rows P (tid % (T / P)) .. +P, k 8 (tid / (T / P)) .. +8
+    template <bool KC>
+    __device__ static __forceinline__ int row_of(int i) {
+        const int tid = threadIdx.x & 255;
+        return KC ? (tid + 256 * i) / CH : P * (tid % (T / P)) + i;
+    }
+    template <bool KC>
+    __device__ static __forceinline__ int k_of(int i) {
+        const int tid = threadIdx.x & 255;
+        return 8 * (KC ? (tid + 256 * i) % CH : tid / (T / P));
+    }
+    // element loads of a ragged step: zeros past K, rows clamped into the matrix
+    template <bool KC>
+    __device__ static __forceinline__ void load_edge(const char* base, int r0, int R, int K, int k0, Patch& p) {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, (long long)R * K * E);
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+        for (int i = 0; i < P; i++) {
+            const int row = min(r0 + row_of<KC>(i), R - 1);
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int n = n0 + wn * 32 + j * 16 + r;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int m = m0 + wm * 32 + i * 16 + 4 * g + v;
-                if (m < M && n < N) Cb[(size_t)m * N + n] = acc[i][j][v];
+            for (int e = 0; e < 8; e++) {
+                const int k = k0 + k_of<KC>(i) + e;
+                const int off = k < K ? (KC ? row * K + k : k * R + row) * E : kOutOfRange;
+                if constexpr (F32) {
+                    p.w[i][e] = __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0);
+                } else {
+                    const uint32_t h = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0);
+                    if (e & 1) p.w[i][e / 2] |= h << 16;
+                    else p.w[i][e / 2] = h;
+                }
             }
         }
+    }
+    // whole patches: every address inside the operand (the caller sends a
+    // step that could leave it to load_edge)
+    template <bool KC>
+    __device__ static __forceinline__ void load(const char* base, int r0, int R, int K, int k0, Patch& p) {
+        typedef uint32_t v4 __attribute__((ext_vector_type(4), aligned(2)));
+        if constexpr (KC) {
+#pragma unroll
+            for (int i = 0; i < P; i++) {
+                const int row = min(r0 + row_of<true>(i), R - 1);
+                const uint32_t off = ((uint32_t)row * K + k0 + k_of<true>(i)) * E;
+#pragma unroll
+                for (int q = 0; q < E / 2; q++) {
+                    const v4 v = *reinterpret_cast<const v4*>(base + off + 16 * q);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) p.w[i][4 * q + e] = v[e];
+                }
+            }
+        } else {
+            // 8 loads of P consecutive elements, transposed in registers
+            constexpr int W = P * E;  // bytes per load
+            typedef uint32_t vw __attribute__((ext_vector_type(W >= 4 ? W / 4 : 1), aligned(2)));
+            int row = r0 + row_of<false>(0);
+            if (row >= R) row = max(R - P, 0);
+            uint32_t v[8][W >= 4 ? W / 4 : 1];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const uint32_t off = ((uint32_t)(k0 + k_of<false>(0) + e) * R + row) * E;
+                if constexpr (W == 2) {
+                    v[e][0] = *reinterpret_cast<const uint16_t*>(base + off);
+                } else if constexpr (W == 4) {
+                    typedef uint32_t u1 __attribute__((aligned(2)));
+                    v[e][0] = *reinterpret_cast<const u1*>(base + off);
+                } else {
+                    const vw x = *reinterpret_cast<const vw*>(base + off);
+#pragma unroll
+                    for (int q = 0; q < W / 4; q++) v[e][q] = x[q];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < P; i++) {
+                if constexpr (F32) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) p.w[i][e] = v[e][i];
+                } else {
+                    // bf16 i of the load: half i & 1 of word i / 2
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        p.w[i][e] = __builtin_amdgcn_perm(v[2 * e + 1][i / 2], v[2 * e][i / 2],
+                                                          (i & 1) ? 0x07060302u : 0x05040100u);
+                }
+            }
+        }
+    }
+    // terms of the patch into LDS
+    template <bool KC>
+    __device__ static __forceinline__ void store(uint16_t* lds, const Patch& p) {
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+            const int row = row_of<KC>(i), c = swz(row, k_of<KC>(i) / 8);
+            uint16_t* dst = lds + row * BK + 8 * c;
+            if constexpr (!F32) {
+                *reinterpret_cast<u32x4*>(dst) = u32x4{p.w[i][0], p.w[i][1], p.w[i][2], p.w[i][3]};
+            } else {
+                u32x4 t[3];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const uint32_t b0 = p.w[i][2 * q], b1 = p.w[i][2 * q + 1];
+                    t[0][q] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+                    const float r0 = __uint_as_float(b0) - __uint_as_float(b0 & 0xffff0000u);
+                    const float r1 = __uint_as_float(b1) - __uint_as_float(b1 & 0xffff0000u);
+                    const uint32_t m0 = __float_as_uint(r0), m1 = __float_as_uint(r1);
+                    t[1][q] = __builtin_amdgcn_perm(m1, m0, 0x07060302u);
+                    const float l0 = r0 - __uint_as_float(m0 & 0xffff0000u);
+                    const float l1 = r1 - __uint_as_float(m1 & 0xffff0000u);
+                    t[2][q] = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)l0) |
+                              ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)l1) << 16);
+                }
+#pragma unroll
+                for (int q = 0; q < 3; q++) *reinterpret_cast<u32x4*>(dst + q * T * BK) = t[q];
+            }
+        }
+    }
+};
+
+// KA / KB: A stored [M][K] (not transA), B stored [N][K] (transB). G groups
+// of 4 waves share a block's tile: group q takes steps q, q + G, ... through
+// LDS stages of its own and the groups' sums are added in order at the end.
+template <int T, int G, int BK, bool KA, bool FA, bool KB, bool FB>
+__global__ __launch_bounds__(256 * G, G <= 2 ? 2 : 1) void k_mm(const void* __restrict__ A, const void* __restrict__ B,
+                                                   float* __restrict__ C, int M, int N, int K, int xcd_map) {
+    using OA = MmOperand<T, BK, FA>;
+    using OB = MmOperand<T, BK, FB>;
+    constexpr int TF = T / 32;  // 16-wide fragments per wave and side
+    constexpr int STAGE = OA::ELEMS + OB::ELEMS;
+    // two LDS stages (one barrier per step) while two blocks still fit a CU
+    constexpr int NS = 2 * G * STAGE * 2 <= (G > 1 ? 144 : 80) * 1024 ? 2 : 1;
+    constexpr size_t kRed = G > 1 ? (size_t)(G - 1) * T * T * 4 : 0;
+    constexpr size_t kLds = (size_t)G * NS * STAGE * 2 > kRed ? (size_t)G * NS * STAGE * 2 : kRed;
+    __shared__ __align__(16) char smem[kLds];
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
+    const int grp = G > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+    uint16_t* lds = reinterpret_cast<uint16_t*>(smem) + grp * NS * STAGE;
+    const int wm = wave >> 1, wn = wave & 1, r = lane & 15, g = lane >> 4;
+    // xcd_map (batches, a one-dimensional grid): blocks are dealt to the 8
+    // XCDs round-robin, and XCD k takes the k-th contiguous run of the tiles
+    // of all batch entries, so that an entry's tiles share its operands in
+    // one L2 (30 x 92 x 725 x 687 ff 46.9 -> 41.7 us; a single product
+    // gains nothing and would pay the divisions, 1024^3 hh 9.5 -> 10.0)
+    int bz = blockIdx.z, m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+    if (xcd_map) {
+        const int gx = (N + T - 1) / T, gy = (M + T - 1) / T;
+        const int items = gridDim.x, q8 = items >> 3, rem8 = items & 7;
+        const int xcd = blockIdx.x & 7;
+        const int item = xcd * q8 + min(xcd, rem8) + ((int)blockIdx.x >> 3);
+        bz = item / (gx * gy);
+        const int t2 = item - bz * (gx * gy);
+        m0 = t2 / gx * T;
+        n0 = t2 % gx * T;
+    }
+    const char* Ab = reinterpret_cast<const char*>(A) + (size_t)bz * M * K * OA::E;
+    const char* Bb = reinterpret_cast<const char*>(B) + (size_t)bz * K * N * OB::E;
+
+    floatx4 acc[TF][TF];
+#pragma unroll
+    for (int i = 0; i < TF; i++)
+#pragma unroll
+        for (int j = 0; j < TF; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    typename OA::Patch pa;
+    typename OB::Patch pb;
+    auto compute = [&](const uint16_t* buf) {
+#pragma unroll
+        for (int kk = 0; kk < BK / 32; kk++) {
+            bf16x8 af[TF][OA::NT];
+#pragma unroll
+            for (int i = 0; i < TF; i++) {
+                const int row = wm * (T / 2) + 16 * i + r;
+#pragma unroll
+                for (int t = 0; t < OA::NT; t++)
+                    af[i][t] = *reinterpret_cast<const bf16x8*>(buf + (t * T + row) * BK + 8 * OA::swz(row, 4 * kk + g));
+            }
+#pragma unroll
+            for (int j = 0; j < TF; j++) {
+                const int row = wn * (T / 2) + 16 * j + r;
+                bf16x8 bfr[OB::NT];
+#pragma unroll
+                for (int t = 0; t < OB::NT; t++)
+                    bfr[t] = *reinterpret_cast<const bf16x8*>(buf + OA::ELEMS + (t * T + row) * BK +
+                                                              8 * OB::swz(row, 4 * kk + g));
+#pragma unroll
+                for (int ta = 0; ta < OA::NT; ta++)
+#pragma unroll
+                    for (int tb = 0; tb < OB::NT; tb++)
+                        if (ta + tb <= 2)
+#pragma unroll
+                            for (int i = 0; i < TF; i++) acc[i][j] = mfma16x16x32(bfr[tb], af[i][ta], acc[i][j]);
+            }
+        }
+    };
+    // steps the whole-patch loads may take: all of K in whole steps, less the
+    // last one when a row-contiguous patch can run past the last row's end
+    // (by fewer than P elements, so by less than a row), none when a row is
+    // shorter than a patch
+    int nf = K / BK;
+    if (K % BK == 0 && ((!KA && M % OA::P) || (!KB && N % OB::P))) nf--;
+    if ((!KA && M < OA::P) || (!KB && N < OB::P)) nf = 0;
+    auto store = [&](uint16_t* buf) {
+        OA::template store<KA>(buf, pa);
+        OB::template store<KB>(buf + OA::ELEMS, pb);
+    };
+    const int ns = (K + BK - 1) / BK;
+    auto load = [&](int s) {
+        if (s < nf) {
+            OA::template load<KA>(Ab, m0, M, K, s * BK, pa);
+            OB::template load<KB>(Bb, n0, N, K, s * BK, pb);
+        } else if (s < ns) {
+            OA::template load_edge<KA>(Ab, m0, M, K, s * BK, pa);
+            OB::template load_edge<KB>(Bb, n0, N, K, s * BK, pb);
+        }
+    };
+    load(grp);
+    if constexpr (NS == 2) {
+        if (grp < ns) store(lds);
+        __syncthreads();
+    }
+    for (int s0 = 0, it = 0; s0 < ns; s0 += G, it++) {
+        const int s = s0 + grp;
+        if constexpr (NS == 2) {
+            load(s + G);
+            if (s < ns) compute(lds + (it & 1) * STAGE);
+            if (s + G < ns) store(lds + ((it + 1) & 1) * STAGE);
+            __syncthreads();
+        } else {
+            if (s < ns) store(lds);
+            __syncthreads();
+            load(s + G);
+            if (s < ns) compute(lds);
+            __syncthreads();  // the step's fragments have been read
+        }
+    }
+    if constexpr (G > 1) {
+        // (the last step's barrier has passed: the stages are free)
+        float4* red = reinterpret_cast<float4*>(smem);
+        const int t = threadIdx.x & 255;
+        if (grp > 0)
+#pragma unroll
+            for (int i = 0; i < TF; i++)
+#pragma unroll
+                for (int j = 0; j < TF; j++)
+                    red[((grp - 1) * TF * TF + i * TF + j) * 256 + t] =
+                        make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int q = 0; q < G - 1; q++)
+#pragma unroll
+            for (int i = 0; i < TF; i++)
+#pragma unroll
+                for (int j = 0; j < TF; j++) {
+                    const float4 v = red[(q * TF * TF + i * TF + j) * 256 + t];
+                    acc[i][j] += floatx4{v.x, v.y, v.z, v.w};
+                }
+    }
+    // lane (r, g): row r, columns 4g .. 4g + 3 of each 16 x 16 fragment
+    float* Cb = C + (size_t)bz * M * N;
+#pragma unroll
+    for (int i = 0; i < TF; i++) {
+        const int m = m0 + wm * (T / 2) + 16 * i + r;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < TF; j++) {
+            const int n = n0 + wn * (T / 2) + 16 * j + 4 * g;
+            float* dst = Cb + (size_t)m * N + n;
+            typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+            if (n + 3 < N) {
+                *reinterpret_cast<f4u*>(dst) = f4u{acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (n + v < N) dst[v] = acc[i][j][v];
+            }
+        }
+    }
+}
+
+template <int T, int G>
+static void launch_mm_t(hipStream_t s, const void* A, const void* B, float* C, int M, int N, int K, int batch,
+                        bool ka, bool fa, bool kb, bool fb) {
+    const unsigned gx = (N + T - 1) / T, gy = (M + T - 1) / T;
+    const int xcd_map = batch > 1 && (long long)gx * gy * batch < (1ll << 22);
+    const dim3 grid = xcd_map ? dim3(gx * gy * batch) : dim3(gx, gy, batch);
+#define GH_MM(KA, FA, KB, FB) \
+    hipLaunchKernelGGL((k_mm<T, G, T == 128 && (FA || FB) ? 32 : 64, KA, FA, KB, FB>), grid, dim3(256 * G), 0, s, A, B, C, M, N, K, xcd_map)
+#define GH_MM_T(KA, KB)                              \
+    do {                                             \
+        if (fa && fb) GH_MM(KA, true, KB, true);     \
+        else if (fa) GH_MM(KA, true, KB, false);     \
+        else if (fb) GH_MM(KA, false, KB, true);     \
+        else GH_MM(KA, false, KB, false);            \
+    } while (0)
+    if (ka && kb) GH_MM_T(true, true);
+    else if (ka) GH_MM_T(true, false);
+    else GH_MM_T(false, false);
+#undef GH_MM_T
+#undef GH_MM
+}
+
+// Tile and K groups, by the number of 64 x 64 tiles n64 of the whole call
+// (256 CUs), measured in HIP graphs (us; T/G, f = f32, h = bf16 operands):
+//   n64 <= 64: 32 x 32 tiles, 4 groups. Few tiles are bound by the chain of
+//     K steps on each: 64 x 64 x 2048 ff 15.1 against 37.6 (64/2), 47.9
+//     (64/1); 1103 x 65 x 1699 ff 14.9 / 33.0 / 42.3; 512^3 hh 3.6 / 4.9 /
+//     5.2; but 128 tiles (8 x 200^2 x 200 fh) 7.2 / 5.9 / 6.6.
+//   n64 <= 256: 64 x 64, 2 groups, one block per CU: 1024^3 hh 9.5 against
+//     11.9 (64/1) and 14.0 (32/4), ff 23.0 / 26.6 / 34.6.
+//   else 64 x 64, 1 group: 2048^3 hh 39.6 against 41.4 (64/2), 45.2 (128/1);
+//     30 x 92 x 725 x 687 ff 41.7 / 50.3 / 50.9.
+//   128 x 128 from 512 such tiles: half the operand traffic, 4096^3 hh 165
+//     against 224 (64/1), fh 398 / 598; 48 x 512 x 512 x 64 ff 20.2 / 20.6.
+// The element-wise gather kernel this replaced: 1024^3 hh 52.4, 48 x 512 x
+// 512 x 64 ff 49.2.
+static void launch_mm(hipStream_t s, const void* A, const void* B, float* C, int M, int N, int K, int batch, bool ka,
+                      bool fa, bool kb, bool fb) {
+    const long long n64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * batch;
+    const long long n128 = (long long)((M + 127) / 128) * ((N + 127) / 128) * batch;
+    if (n64 <= 64) launch_mm_t<32, 4>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
+    else if (n64 <= 256) launch_mm_t<64, 2>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
+    else if (n128 < 512) launch_mm_t<64, 1>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
+    else launch_mm_t<128, 1>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
 }
 
 static bool linear_fast_ok(const void* x, const void* W, int K) {
@@ -248,14 +493,9 @@ int matmul_dt_raw(hipStream_t s, const void* A, const void* B, float* C, uint32_
         set_error("gorch_hip_matmul_dt: an operand of one batch entry is 2 GiB or more");
         return GORCH_HIP_EUNSUPPORTED;
     }
-    const dim3 grid((N + 63) / 64, (M + 63) / 64, batch);
-    const int tA = transA ? 1 : 0, tB = transB ? 1 : 0, m = (int)M, n = (int)N, k = (int)K;
-    if (aBF16 && bBF16) hipLaunchKernelGGL((k_matmul_mfma<1, 1>), grid, dim3(256), 0, s, A, B, C, m, n, k, tA, tB);
-    else if (aBF16) hipLaunchKernelGGL((k_matmul_mfma<1, 3>), grid, dim3(256), 0, s, A, B, C, m, n, k, tA, tB);
-    else if (bBF16) hipLaunchKernelGGL((k_matmul_mfma<3, 1>), grid, dim3(256), 0, s, A, B, C, m, n, k, tA, tB);
-    else hipLaunchKernelGGL((k_matmul_mfma<3, 3>), grid, dim3(256), 0, s, A, B, C, m, n, k, tA, tB);
+    launch_mm(s, A, B, C, (int)M, (int)N, (int)K, (int)batch, !transA, !aBF16, transB != 0, !bBF16);
     count(CNT_GENERIC_MATMUL);
-    return check_launch("matmul_mfma");
+    return check_launch("matmul");
 }
 
 }  // namespace gh
