@@ -463,51 +463,96 @@ __global__ __launch_bounds__(NW * 64) void k_attn_rows(AttnArgs a) {
 // causal case, nn/attention.go:64-145, as the cached path's prompt pass) on
 // the f32 matrix cores (v_mfma_f32_16x16x4_f32: products and sums in f32).
 //
-// A block of NW waves takes 16 * NW consecutive query rows of one (sequence,
-// head); wave w owns 16 of them. Keys stream through LDS in stages of KT:
-// K row-major [key][dim] and V transposed [dim][key], loaded once per block
-// for all its waves. Per 16-key slice a wave computes S^T = K Q^T (lane
-// (r, g) then holds keys 4g .. 4g+3 of query r), applies the scale
-// ((q.k) * scale, as the reference), the causal mask and an online softmax
-// per query (running max m and per-lane partial sums l rescaled by
-// exp(m_old - m_new)), and accumulates O^T += V^T P^T: the probabilities are
-// already in the B-operand position when the MFMA's k index runs over the
-// keys a lane holds, so P never leaves registers. O = O^T / l at the end
-// (the reference normalises P before P.V: same values up to rounding).
-// The dims of the QK^T product are visited as 16u + 4g + c by (step, lane
-// group), so both Q and K fragments are 16-byte reads.
+// Bound by the f32 matrix cores (64 FLOP/clock and SIMD; 2.5 GFLOP at 777
+// rows of 16 heads of 128 take 18 us on all CUs) and by the longest chain:
+// a wave that walked all 777 keys for its 16 rows would take 46 us alone. So
+// a block of 8 waves takes 32 query rows (row group w & 1) and splits each
+// 64-key stage over 4 key groups (w >> 1), whose online softmax states are
+// merged in key-group order at the end; blocks go out longest first. With
+// an even number of query heads per KV head the two row groups are 16 rows
+// of two heads that share the staged keys. 777 rows, 16 / 8 heads of 128:
+// 160 us with 128 rows per block and no key groups, 45 us so; 16 x 512 rows,
+// 25 heads of 64: 330 -> 214 us (63 TFLOP/s; the softmax between the two
+// products is what the matrix cores wait for).
+//
+// K and V stages go straight from the cache to LDS (raw buffer loads to LDS,
+// 16 bytes a lane, rows past the end zero), row-major, the stage after next
+// to come issued behind the barrier that frees its buffer: one barrier per
+// stage. 16-byte chunk c of row k sits at c ^ (k & 15), which keeps both the
+// 16-byte K fragment reads and the V element reads free of bank conflicts.
+//
+// Per 16-key slice a wave computes S^T = K Q^T (lane (r, g) then holds keys
+// 4g .. 4g+3 of query r), applies the scale ((q.k) * scale, as the
+// reference), the causal mask and an online softmax per query (running max
+// m and per-lane partial sums l rescaled by exp(m_old - m_new)), and
+// accumulates O^T += V^T P^T: the probabilities are already in the B-operand
+// position when the MFMA's k index runs over the keys a lane holds, so P
+// never leaves registers. O = O^T / l at the end (the reference normalises P
+// before P.V: same values up to rounding). The dims of the QK^T product are
+// visited as 16u + 4g + c by (step, lane group), so both Q and K fragments
+// are 16-byte reads.
 __device__ __forceinline__ floatx4 mfma_f32x4(float a, float b, const floatx4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-template <int HD, int NW>
-__global__ __launch_bounds__(NW * 64) void k_attn_flash(AttnArgs a) {
-    constexpr int KT = 32;   // keys per LDS stage
-    constexpr int QU = HD / 16;
-    __shared__ float4 Ks[KT][HD / 4 + 1];   // K[key][dims 4c..4c+3]
-    __shared__ float4 Vt[HD][KT / 4 + 1];   // V^T[dim][keys 4c..4c+3]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = lane & 15, g = lane >> 4;
-    const int b = blockIdx.z, h = blockIdx.y;
-    const int qbase = blockIdx.x * 16 * NW;
-    const int qi = qbase + wave * 16 + r;  // this lane's query (column of S^T)
-    const int pos = a.pos_dev ? *a.pos_dev : a.pos_host;
-    const int kvh = a.kv_heads ? h / ((int)gridDim.y / a.kv_heads) : h;
-    const int kvd = a.kv_dim ? a.kv_dim : a.dim;
-    const size_t cbase = (size_t)b * a.max_seq * kvd + (size_t)kvh * HD;
-    const float4* K4 = reinterpret_cast<const float4*>(a.kc + cbase);
-    const float4* V4 = reinterpret_cast<const float4*>(a.vc + cbase);
-    const int kvd4 = kvd >> 2;
-    const int t_all = pos + a.new_seq;
-    const int qlast = min(a.new_seq, qbase + 16 * NW) - 1;
-    const int kend = a.causal ? pos + qlast + 1 : t_all;
+constexpr int kFlashKeys = 64;  // keys per stage
 
+// One stage buffer: K then V, [key][HD] floats, chunks swizzled.
+template <int HD>
+struct FlashStage {
+    static constexpr int kFloats = 2 * kFlashKeys * HD;
+    // the block's 8 waves copy keys k0 .. k0 + 63 of K and V; keys from
+    // t_all on read as zeros
+    __device__ static __forceinline__ void issue(float* buf, __amdgpu_buffer_rsrc_t rk, __amdgpu_buffer_rsrc_t rv,
+                                                 int k0, int t_all, int kvd) {
+        constexpr int CPR = HD / 4, RPI = 64 / CPR;           // chunks per row, rows per wave load
+        constexpr int N = kFlashKeys / RPI / 8;               // loads per wave and operand
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const int row0 = (wave * N + i) * RPI, row = row0 + lane / CPR, key = k0 + row;
+            const int off = key < t_all ? key * kvd * 4 + ((lane % CPR) ^ (row & 15)) * 16 : kOutOfRange;
+            typedef __attribute__((address_space(3))) void* lds_ptr;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr)(buf + row0 * HD), 16, off, 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr)(buf + (kFlashKeys + row0) * HD), 16, off, 0, 0, 0);
+        }
+    }
+};
+
+template <int HD>
+__global__ __launch_bounds__(512) void k_attn_flash(AttnArgs a, int heads, int pair) {
+    constexpr int QU = HD / 16;
+    // one array per stage, so that reads of one are known not to wait for
+    // the loads into the other
+    __shared__ __align__(16) float st0[FlashStage<HD>::kFloats];
+    __shared__ __align__(16) float st1[FlashStage<HD>::kFloats];
+    __shared__ float red[2][4][2][16];  // [row group][key group][m, l][query]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rg = wave & 1, kg = wave >> 1, r = lane & 15, g = lane >> 4;
+    const int b = blockIdx.z, tile = gridDim.y - 1 - blockIdx.y;
+    // pair: rows of two heads of one KV head, else 32 rows of one head
+    const int h = pair ? 2 * (int)blockIdx.x + rg : (int)blockIdx.x;
+    const int q0 = pair ? tile * 16 : tile * 32 + rg * 16;  // the wave's first query row
+    const int qlast = min(a.new_seq, tile * (pair ? 16 : 32) + (pair ? 16 : 32)) - 1;
+    const int qi = q0 + r;                                   // this lane's query (column of S^T)
+    const int pos = a.pos_dev ? *a.pos_dev : a.pos_host;
+    const int kvh = a.kv_heads ? h / (heads / a.kv_heads) : h;
+    const int kvd = a.kv_dim ? a.kv_dim : a.dim;
+    const size_t cbase = (size_t)b * a.max_seq * kvd + (size_t)__builtin_amdgcn_readfirstlane(kvh) * HD;
+    const int t_all = pos + a.new_seq;
+    const int kend = a.causal ? pos + qlast + 1 : t_all;
+    // the last key any of the wave's queries sees
+    const int kwave = a.causal ? min(t_all, pos + q0 + 16) : (q0 < a.new_seq ? t_all : 0);
+    const long long span = ((long long)(t_all - 1) * kvd + HD) * 4;
+    const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.kc + cbase, span);
+    const __amdgpu_buffer_rsrc_t rv = make_rsrc(a.vc + cbase, span);
+
+    FlashStage<HD>::issue(st0, rk, rv, 0, t_all, kvd);
     const bool qok = qi < a.new_seq;
     const float* qrow = a.q + (size_t)(b * a.new_seq + (qok ? qi : 0)) * a.q_stride + h * HD;
     float4 qf[QU];
 #pragma unroll
-    for (int u = 0; u < QU; u++)
-        qf[u] = qok ? *reinterpret_cast<const float4*>(qrow + 16 * u + 4 * g) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int u = 0; u < QU; u++) qf[u] = *reinterpret_cast<const float4*>(qrow + 16 * u + 4 * g);
     const int P = pos + qi;  // absolute position of this lane's query
 
     floatx4 o[QU];
@@ -515,78 +560,101 @@ __global__ __launch_bounds__(NW * 64) void k_attn_flash(AttnArgs a) {
     for (int t = 0; t < QU; t++) o[t] = floatx4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;
 
-    for (int k0 = 0; k0 < kend; k0 += KT) {
-        __syncthreads();  // the previous stage has been read
-        for (int i = threadIdx.x; i < KT * HD / 4; i += NW * 64) {
-            const int kr = i / (HD / 4), c4 = i - kr * (HD / 4);
-            const int key = k0 + kr;
-            float4 kv = make_float4(0.f, 0.f, 0.f, 0.f), vv = kv;
-            if (key < t_all) {
-                kv = K4[(size_t)key * kvd4 + c4];
-                vv = V4[(size_t)key * kvd4 + c4];
-            }
-            Ks[kr][c4] = kv;
-            float* vt = reinterpret_cast<float*>(&Vt[0][0]);
-            constexpr int VS = 4 * (KT / 4 + 1);  // floats per V^T row
-            vt[(4 * c4 + 0) * VS + kr] = vv.x;
-            vt[(4 * c4 + 1) * VS + kr] = vv.y;
-            vt[(4 * c4 + 2) * VS + kr] = vv.z;
-            vt[(4 * c4 + 3) * VS + kr] = vv.w;
+    auto slice = [&](const float* buf, int k0) {
+        const float* Ks = buf + (kg * 16 + r) * HD;
+        const int voff = (kFlashKeys + kg * 16 + 4 * g) * HD;
+        floatx4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < QU; u++) {
+            const float4 kf = *reinterpret_cast<const float4*>(Ks + 4 * ((4 * u + g) ^ r));
+            s = mfma_f32x4(kf.x, qf[u].x, s);
+            s = mfma_f32x4(kf.y, qf[u].y, s);
+            s = mfma_f32x4(kf.z, qf[u].z, s);
+            s = mfma_f32x4(kf.w, qf[u].w, s);
         }
-        __syncthreads();
+        float sv[4];
+        float tmax = -INFINITY;
 #pragma unroll
-        for (int sub = 0; sub < KT / 16; sub++) {
-            floatx4 s = {0.f, 0.f, 0.f, 0.f};
+        for (int v = 0; v < 4; v++) {
+            const int key = k0 + kg * 16 + 4 * g + v;
+            const bool ok = key < t_all && (!a.causal || key <= P);
+            sv[v] = ok ? s[v] * a.scale : -INFINITY;
+            tmax = fmaxf(tmax, sv[v]);
+        }
+        // the query's maximum over the 4 lane groups holding its keys
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+        const float mnew = fmaxf(m, tmax);
+        const float alpha = mnew == -INFINITY ? 1.f : expf(m - mnew);
+        float p[4], psum = 0.f;
 #pragma unroll
-            for (int u = 0; u < QU; u++) {
-                const float4 kf = Ks[sub * 16 + r][4 * u + g];
-                s = mfma_f32x4(kf.x, qf[u].x, s);
-                s = mfma_f32x4(kf.y, qf[u].y, s);
-                s = mfma_f32x4(kf.z, qf[u].z, s);
-                s = mfma_f32x4(kf.w, qf[u].w, s);
-            }
-            float sv[4];
-            float tmax = -INFINITY;
+        for (int v = 0; v < 4; v++) {
+            p[v] = sv[v] == -INFINITY ? 0.f : expf(sv[v] - mnew);
+            psum += p[v];
+        }
+        l = l * alpha + psum;
+        m = mnew;
+#pragma unroll
+        for (int t = 0; t < QU; t++) {
+            o[t] *= alpha;
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int key = k0 + sub * 16 + 4 * g + v;
-                const bool ok = qok && key < t_all && (!a.causal || key <= P);
-                sv[v] = ok ? s[v] * a.scale : -INFINITY;
-                tmax = fmaxf(tmax, sv[v]);
-            }
-            // the query's maximum over the 4 lane groups holding its keys
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-            const float mnew = fmaxf(m, tmax);
-            const float alpha = mnew == -INFINITY ? 1.f : expf(m - mnew);
-            float p[4], psum = 0.f;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                p[v] = sv[v] == -INFINITY ? 0.f : expf(sv[v] - mnew);
-                psum += p[v];
-            }
-            l = l * alpha + psum;
-            m = mnew;
-#pragma unroll
-            for (int t = 0; t < QU; t++) {
-                o[t] *= alpha;
-                const float4 vf = Vt[16 * t + r][4 * sub + g];
-                o[t] = mfma_f32x4(vf.x, p[0], o[t]);
-                o[t] = mfma_f32x4(vf.y, p[1], o[t]);
-                o[t] = mfma_f32x4(vf.z, p[2], o[t]);
-                o[t] = mfma_f32x4(vf.w, p[3], o[t]);
+                // V[key 4g + v][dim 16t + r]
+                const float vf = buf[voff + v * HD + (((16 * t + (r & 12)) ^ (16 * g + 4 * v)) | (r & 3))];
+                o[t] = mfma_f32x4(vf, p[v], o[t]);
             }
         }
+    };
+    // stage s is computed from one buffer while stage s + 1 lands in the
+    // other: the barrier says that every wave's part of stage s has arrived
+    // and that the other buffer has been read
+    auto stage = [&](float* cur, float* nxt, int k0) {
+        block_sync_dma();
+        if (k0 + kFlashKeys < kend) FlashStage<HD>::issue(nxt, rk, rv, k0 + kFlashKeys, t_all, kvd);
+        if (k0 + kg * 16 < kwave) slice(cur, k0);
+    };
+    for (int k0 = 0; k0 < kend; k0 += 2 * kFlashKeys) {
+        stage(st0, st1, k0);
+        if (k0 + kFlashKeys < kend) stage(st1, st0, k0 + kFlashKeys);
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
+    // merge the 4 key groups: common maximum, then the rescaled sums
+    if (g == 0) {
+        red[rg][kg][0][r] = m;
+        red[rg][kg][1][r] = l;
+    }
+    __syncthreads();
+    float M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) M = fmaxf(M, red[rg][k][0][r]);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float mk = red[rg][k][0][r];
+        L += mk == -INFINITY ? 0.f : red[rg][k][1][r] * expf(mk - M);
+    }
+    const float sc = m == -INFINITY ? 0.f : expf(m - M);
+    // (every wave has left the stages: the barrier above)
+    float4* mo = reinterpret_cast<float4*>(st0);  // [row group][key group][t][lane]
+    static_assert(8 * QU * 64 * 4 <= FlashStage<HD>::kFloats, "merge buffer");
+#pragma unroll
+    for (int t = 0; t < QU; t++)
+        mo[((rg * 4 + kg) * QU + t) * 64 + lane] = make_float4(o[t][0] * sc, o[t][1] * sc, o[t][2] * sc, o[t][3] * sc);
+    __syncthreads();
     if (qok) {
         const int orow = b * a.new_seq + qi;
-        const float inv = 1.0f / l;
+        const float inv = 1.0f / L;
 #pragma unroll
-        for (int t = 0; t < QU; t++)
-            attn_out4(a, orow, h * HD + 16 * t + 4 * g,
-                      make_float4(o[t][0] * inv, o[t][1] * inv, o[t][2] * inv, o[t][3] * inv));
+        for (int tt = 0; tt < QU / 4; tt++) {
+            const int t = kg * (QU / 4) + tt;
+            float4 s = mo[(rg * 4 * QU + t) * 64 + lane];
+#pragma unroll
+            for (int k = 1; k < 4; k++) {
+                const float4 v = mo[((rg * 4 + k) * QU + t) * 64 + lane];
+                s = make_float4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w);
+            }
+            attn_out4(a, orow, h * HD + 16 * t + 4 * g, make_float4(s.x * inv, s.y * inv, s.z * inv, s.w * inv));
+        }
     }
 }
 
@@ -1079,8 +1147,14 @@ static AttnRoute attn_route(const AttnArgs& a, int heads, int rows) {
     const long long visible = a.pos_dev ? (long long)a.max_seq : (long long)a.pos_host + a.new_seq;
     const bool lds_ok = (size_t)visible * sizeof(float) <= kAttnMaxLdsBytes;
     const int blocks = heads * rows;
-    // new rows per sequence from which the matrix-core prefill kernel runs
-    constexpr int flash_min = 32;
+    // The matrix-core prefill kernel: from 32 new rows per sequence, or from
+    // 4 when the one-block-per-(head, row) kernels would need 1536 blocks
+    // and more, each reading the whole cache (us, flash against those: 4
+    // sequences of 16 rows, 25 heads, 316 keys, 1600 blocks 12.5 / 23.0; 16
+    // of 5, 2000 blocks, 505 keys 31.8 / 75.8; but 4 of 4, 400 blocks 7.5 /
+    // 6.8, and 20 rows of one sequence of 16 heads over 1020 keys, 320
+    // blocks, 50 / 22.5: few rows leave most of a 32-row tile empty).
+    const bool many_rows = a.new_seq >= 32 || (a.new_seq >= 4 && blocks >= 1536);
     const bool aligned = (a.q_stride % 4 == 0) && (a.dim % 4 == 0) && ((a.kv_dim ? a.kv_dim : a.dim) % 4 == 0) &&
                          ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.kc) |
                            reinterpret_cast<uintptr_t>(a.vc) | reinterpret_cast<uintptr_t>(a.out)) % 16 == 0);
@@ -1090,7 +1164,7 @@ static AttnRoute attn_route(const AttnArgs& a, int heads, int rows) {
     };
     // split QKV partials: only the two-pass kernel adds them
     if (a.qkv_part) return cached();
-    if (aligned && a.new_seq >= flash_min && (a.hd == 64 || a.hd == 128)) return kRouteFlash;
+    if (aligned && many_rows && (a.hd == 64 || a.hd == 128)) return kRouteFlash;
     // one row over few heads: each head's keys over several CUs
     if (aligned && blocks < 128 && attn_split_chunks(a, heads, rows)) return kRouteSplit;
     if (aligned && a.max_seq <= 256 && (a.hd == 64 || a.hd == 128 || a.hd == 32 || a.hd == 16))
@@ -1157,12 +1231,12 @@ int launch_attn_cached(hipStream_t s, const AttnArgs& a, int heads, int rows) {
     }
     switch (route) {
         case kRouteFlash: {
-            // many new rows per sequence (prefill): the matrix-core kernel,
-            // 128 query rows per block sharing each staged K/V tile
+            // many new rows per sequence (prefill): the matrix-core kernel
             const int batch = rows / a.new_seq;
-            const dim3 fg((a.new_seq + 127) / 128, heads, batch);
-            if (a.hd == 64) hipLaunchKernelGGL((k_attn_flash<64, 8>), fg, dim3(512), 0, s, a);
-            else hipLaunchKernelGGL((k_attn_flash<128, 8>), fg, dim3(512), 0, s, a);
+            const int pair = a.kv_heads && (heads / a.kv_heads) % 2 == 0;
+            const dim3 fg(pair ? heads / 2 : heads, pair ? (a.new_seq + 15) / 16 : (a.new_seq + 31) / 32, batch);
+            if (a.hd == 64) hipLaunchKernelGGL((k_attn_flash<64>), fg, dim3(512), 0, s, a, heads, pair);
+            else hipLaunchKernelGGL((k_attn_flash<128>), fg, dim3(512), 0, s, a, heads, pair);
             count(CNT_ATTENTION);
             return check_launch("attn_flash");
         }

@@ -481,6 +481,17 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, long 
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, n, 0x00020000);
 }
 constexpr int kOutOfRange = 0x7fff0000;  // an offset past any resource (+ small immediates)
+// Barrier for stages filled by loads to LDS: this wave's loads have landed
+// (vmcnt 0) and its LDS reads are done (lgkmcnt 0), then the block's waves
+// meet. Unlike __syncthreads it is no fence, so loads the next stage issues
+// stay in flight; the empty asm keeps the compiler from moving memory
+// accesses across it.
+__device__ __forceinline__ void block_sync_dma() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
 // Cache policy (the buffer loads' aux bits) for data a launch reads once and
 // the next launches do not reuse: GEMV weights, K/V cache rows. 2 is the nt
 // (non-temporal) bit; measured faster than the default policy for every
