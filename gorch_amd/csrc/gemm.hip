@@ -2,17 +2,17 @@
 //   C[m,n] = residual[m,n] + epi( sum_k A[m,k] * W[n,k] + bias[n] )
 // with A f32 [M,K], W bf16 [N,K] (the nn.Linear layout, nn/module.go:61-88).
 //
-// Two kernels, both staging 64-wide K steps of A (converted from f32 as it
-// is written to LDS) and W through LDS into v_mfma_f32_16x16x32_bf16:
-//   k_gemm_bf16w: 128 x 128 tiles of 4 waves (2 x 2 waves of 64 x 64), for
-//     problems with at least 256 such tiles (long prefills);
+// Three kernels on v_mfma_f32_16x16x32_bf16, chosen by estimated time
+// (gemm_kind):
+//   k_gemm_kw: few tiles (short prompts, narrow weights): the waves of a block
+//     split K, each through LDS stages of its own;
 //   k_gemm_db: 64-row tiles of 64, 96 or 128 columns on 2 x (2..4) waves of
-//     32 x 32, double-buffered LDS, for the few-tile shapes of a short
-//     prefill (512 x 768 x 2304: 72 tiles of 128 x 128).
-// Later steps' global loads (raw buffer loads, no branches) are issued into
-// registers before the current step's MFMAs so memory latency overlaps the
-// math. LDS rows are padded to 160 bytes, which makes the 16-byte fragment
-// reads conflict-free on gfx950 (a 144-byte row measured 2-way conflicted).
+//     32 x 32, double-buffered LDS filled through registers;
+//   k_gemm_pp: many tiles (long prompts): 256 x (32 TN) tiles on 8 waves, the
+//     two waves of a SIMD half a step apart.
+// k_gemm_db's LDS rows are padded to 160 bytes, which makes the 16-byte
+// fragment reads conflict-free on gfx950 (a 144-byte row measured 2-way
+// conflicted); the other two load straight to LDS and swizzle instead.
 //
 // Activation modes:
 //   split (default): A = hi + lo in bf16 (two MFMAs per fragment pair),
@@ -20,6 +20,10 @@
 //     widen + f32 sgemm (bf16_matmul.go:166-173);
 //   bf16 (GORCH_HIP_LINEAR_ACT_BF16): A rounded to bf16 (RNE), one MFMA —
 //     the bf16 x bf16 -> f32 MPSGraph path (metal/shim.m:808-857).
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
 #include "common.h"
 
 namespace gh {
@@ -120,185 +124,7 @@ __device__ __forceinline__ void gemm_epilogue(floatx4 (&acc)[TM][TN], const floa
     }
 }
 
-template <int BM, int BN, bool SPLIT, int PF, bool KT>
-__global__ __launch_bounds__(256) void k_gemm_bf16w(const float* __restrict__ A, const uint16_t* __restrict__ W,
-                                                    const float* __restrict__ bias, const float* residual,
-                                                    OutDesc od, int M, int N, int K, int epilogue) {
-    constexpr int NA = SPLIT ? 2 : 1;
-    constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
-    constexpr int A_F4 = BM * kBK / 4 / 256;  // float4 loads of A per thread
-    constexpr int W_U4 = BN * kBK / 8 / 256;  // uint4 loads of W per thread
-    __shared__ __align__(16) uint16_t As[NA][BM][kLDA];
-    __shared__ __align__(16) uint16_t Ws[BN][kLDA];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-
-    // PF register stages: the loads of K-step i + PF are issued as soon as
-    // step i has been written to LDS, so PF steps of latency are in flight.
-    // Raw buffer loads over the block's rows, branch-free: rows past M or N
-    // are clamped into the tile (computed, never stored) and a K-tail chunk
-    // gets an out-of-range offset, which reads as zeros. (A load under a
-    // branch makes the compiler drain every outstanding load before each
-    // LDS store, so no prefetch would survive a step.)
-    const int mrows = min(BM, M - m0), ncols = min(BN, N - n0);
-    const __amdgpu_buffer_rsrc_t rsa = make_rsrc(A + (size_t)m0 * K, (long long)mrows * K * 4);
-    const __amdgpu_buffer_rsrc_t rsw = make_rsrc(W + (size_t)n0 * K, (long long)ncols * K * 2);
-    float4 ra[PF][A_F4];
-    uint4 rw[PF][W_U4];
-    auto gload = [&](int k0, float4 (&a)[A_F4], uint4 (&wv)[W_U4]) {
-#pragma unroll
-        for (int i = 0; i < A_F4; i++) {
-            const int idx = tid + 256 * i, row = idx >> 4, c4 = idx & 15;
-            const int k = k0 + 4 * c4;
-            const int off = (!KT || k < K) ? (min(row, mrows - 1) * K + k) * 4 : kOutOfRange;
-            a[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsa, off, 0, 0));
-        }
-#pragma unroll
-        for (int i = 0; i < W_U4; i++) {
-            const int idx = tid + 256 * i, row = idx >> 3, c8 = idx & 7;
-            const int k = k0 + 8 * c8;
-            const int off = (!KT || k < K) ? (min(row, ncols - 1) * K + k) * 2 : kOutOfRange;
-            wv[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsw, off, 0, 0));
-        }
-    };
-    auto sstore = [&](const float4 (&a)[A_F4], const uint4 (&wv)[W_U4]) {
-#pragma unroll
-        for (int i = 0; i < A_F4; i++) {
-            const int idx = tid + 256 * i, row = idx >> 4, c4 = idx & 15;
-            const float f[4] = {a[i].x, a[i].y, a[i].z, a[i].w};
-            uint16_t hi[4], lo[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                if (SPLIT) {
-                    uint32_t u = __float_as_uint(f[e]) & 0xffff0000u;
-                    hi[e] = (uint16_t)(u >> 16);
-                    lo[e] = __builtin_bit_cast(uint16_t, (__bf16)(f[e] - __uint_as_float(u)));
-                } else {
-                    hi[e] = __builtin_bit_cast(uint16_t, (__bf16)f[e]);
-                }
-            }
-            uint2 h2 = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
-            *reinterpret_cast<uint2*>(&As[0][row][4 * c4]) = h2;
-            if (SPLIT) {
-                uint2 l2 = make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
-                *reinterpret_cast<uint2*>(&As[NA - 1][row][4 * c4]) = l2;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < W_U4; i++) {
-            const int idx = tid + 256 * i, row = idx >> 3, c8 = idx & 7;
-            *reinterpret_cast<uint4*>(&Ws[row][8 * c8]) = wv[i];
-        }
-    };
-
-    floatx4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-    const int r = lane & 15, g = lane >> 4;
-    // the epilogue's bias values, loaded while the main loop runs
-    float bn[TN];
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-        const int n = n0 + wn * WN + j * 16 + r;
-        bn[j] = (bias && n < N) ? bias[n] : 0.f;
-    }
-    // the step count is padded to a multiple of PF (padding steps read
-    // zeros) so the loop body has no branch around its loads
-    const int nk = (K + kBK - 1) / kBK;
-    const int nkp = (nk + PF - 1) / PF * PF;
-    // issue the stages in order: the loop waits for stage s while later
-    // stages stay in flight (memory counters complete in issue order), and
-    // the scheduler would otherwise interleave the prologue's loads
-#pragma unroll
-    for (int s = 0; s < PF; s++) {
-        gload(s * kBK, ra[s], rw[s]);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    for (int it0 = 0; it0 < nkp; it0 += PF) {
-#pragma unroll
-        for (int s = 0; s < PF; s++) {
-            const int it = it0 + s;
-            __syncthreads();  // previous step's fragment reads are done
-            sstore(ra[s], rw[s]);
-            __syncthreads();
-            gload((it + PF) * kBK, ra[s], rw[s]);
-#pragma unroll
-            for (int kk = 0; kk < kBK; kk += 32) {
-                bf16x8 bfr[TN];
-#pragma unroll
-                for (int j = 0; j < TN; j++)
-                    bfr[j] = *reinterpret_cast<const bf16x8*>(&Ws[wn * WN + j * 16 + r][kk + 8 * g]);
-#pragma unroll
-                for (int i = 0; i < TM; i++) {
-                    const bf16x8 ahi = *reinterpret_cast<const bf16x8*>(&As[0][wm * WM + i * 16 + r][kk + 8 * g]);
-#pragma unroll
-                    for (int j = 0; j < TN; j++) acc[i][j] = mfma16x16x32(ahi, bfr[j], acc[i][j]);
-                    if (SPLIT) {
-                        const bf16x8 alo =
-                            *reinterpret_cast<const bf16x8*>(&As[NA - 1][wm * WM + i * 16 + r][kk + 8 * g]);
-#pragma unroll
-                        for (int j = 0; j < TN; j++) acc[i][j] = mfma16x16x32(alo, bfr[j], acc[i][j]);
-                    }
-                }
-            }
-        }
-    }
-
-    // Epilogue. Stores and loads share one memory counter, so a loaded value
-    // first used after a store makes that use wait for the store's write
-    // too (and, past a branch, for every store before it): the position and
-    // the residual are loaded and every output value computed before the
-    // first store.
-    const int pos = __builtin_amdgcn_readfirstlane(od.pos_dev ? *od.pos_dev : 0);
-    float res[TM][TN][4];
-    if (residual) {
-        const __amdgpu_buffer_rsrc_t rsr = make_rsrc(residual + (size_t)m0 * N, (long long)mrows * N * 4);
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const int n = n0 + wn * WN + j * 16 + r;
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int ml = wm * WM + i * 16 + 4 * g + v;
-                    const int off = (n < N && ml < mrows) ? (ml * N + n) * 4 : kOutOfRange;
-                    res[i][j][v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsr, off, 0, 0));
-                }
-            }
-    }
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                float s = acc[i][j][v];
-                if (bias) s = s + bn[j];
-                if (epilogue == GORCH_HIP_EPI_GELU) s = gelu_tanh(s);
-                if (residual) s = res[i][j][v] + s;
-                acc[i][j][v] = s;
-            }
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-        const int n = n0 + wn * WN + j * 16 + r;
-        const OutDesc::Col c = od.col(min(n, N - 1), pos);
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int m = m0 + wm * WM + i * 16 + 4 * g + v;
-                if (m < M && n < N) *od.row(c, m) = acc[i][j][v];
-            }
-    }
-}
-
-// Linear for M > 16 when 128 x 128 tiles would not fill the chip (prefill of
-// a few hundred rows: 512 x 768 x {2304, 3072} gives 72..96 such tiles):
+// Linear for a few hundred rows (512 x 768 x {2304, 3072}):
 // 64 x BN tiles (BN = 32 * WGN) on 2 x WGN waves, each wave a 32 x 32
 // sub-tile of 2 x 2 MFMA accumulators. The block's A and W K-steps (64
 // wide) go global -> registers -> one of two LDS stage buffers, so each
@@ -437,6 +263,447 @@ __global__ __launch_bounds__(128 * WGN) void k_gemm_db(const float* __restrict__
     gemm_epilogue<TM, TN, EPI>(acc, bn, residual, od, pos, M, N, m0, mrows, wm * 32, n0 + wn * 32, r, g);
 }
 
+// ---------------------------------------------------------------------------
+// Stages loaded straight to LDS (raw buffer loads to LDS, 16 bytes a lane).
+//
+// A stage is BK = 32 wide: A rows stay f32 (128 bytes, 8 chunks of 16) and
+// are split into their bf16 terms as a fragment is read (f32 and hi + lo take
+// the same LDS), W rows are bf16 (64 bytes, 4 chunks). Chunk c of A row i
+// sits at c ^ (i & 7), of W row i at c ^ ((i >> 1) & 3): conflict-free
+// 16-byte fragment reads. Rows past the tile's edge are clamped into it and
+// chunks past K read as zeros (an out-of-range offset), so steps past the
+// last one cost no traffic.
+constexpr int kStK = 32;
+
+// Lane l of a load takes row l / CH of its group of 64 / CH rows and the
+// chunk that belongs at position l % CH of that row; `chunk` is the same for
+// every group, so a lane's offset is a constant plus a scalar (group row,
+// step). Everything goes through the checked offset: rows past the resource
+// and a step past the last one (kbyte = kOutOfRange) read as zeros, and so do
+// chunks past K when `tail` is kOutOfRange for the lane (0 otherwise).
+template <int CH>
+struct StageLane {
+    int chunk, off;
+    __device__ __forceinline__ StageLane(int lane, int ld) {
+        const int row = lane / CH;
+        chunk = (lane % CH) ^ (CH == 8 ? row : ((row >> 1) & 3));
+        off = row * ld + 16 * chunk;
+    }
+    // copies ROWS rows (stride ld bytes) of the step at byte kbyte to LDS
+    template <int ROWS, bool KT>
+    __device__ __forceinline__ void issue(char* lds, __amdgpu_buffer_rsrc_t rs, int ld, int kbyte, int tail) const {
+        constexpr int RPI = 64 / CH;
+#pragma unroll
+        for (int i = 0; i < ROWS / RPI; i++) {
+            unsigned o = (unsigned)off + (unsigned)(i * RPI * ld + kbyte);
+            if constexpr (KT) o = max(o, (unsigned)tail);
+            typedef __attribute__((address_space(3))) void* lds_ptr;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)(lds + i * 1024), 16, (int)o, 0, 0, 0);
+        }
+    }
+};
+
+// the bf16 terms of 8 consecutive f32 of an A row: hi (truncated) and lo
+// (the remainder rounded), or one rounded term
+template <bool SPLIT>
+__device__ __forceinline__ void a_terms(const float4& u, const float4& v, bf16x8& hi, bf16x8& lo) {
+    const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+    if constexpr (SPLIT) {
+        u32x4 h;
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            h[q] = __builtin_amdgcn_perm(__float_as_uint(f[2 * q + 1]), __float_as_uint(f[2 * q]), 0x07060302u);
+        hi = __builtin_bit_cast(bf16x8, h);
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            lo[e] = (__bf16)(f[e] - __uint_as_float(__float_as_uint(f[e]) & 0xffff0000u));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) hi[e] = (__bf16)f[e];
+    }
+}
+
+// Epilogue of 4 consecutive columns n .. n + 3 of one row at a time (the
+// accumulator layout of (W fragment) x (A fragment) products). Bias and
+// residual come through buffer resources (columns past N or rows past the
+// tile read zeros or a neighbour, never stored); `put` writes the columns
+// below N through the output descriptor.
+struct Out4 {
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    const OutDesc& od;
+    __amdgpu_buffer_rsrc_t rb, rr;
+    int m0, pos, M, N;
+    bool flat, seg4;
+    // rows m0 .. m0 + mrows; seg4: every output segment starts at a multiple
+    // of 4 columns
+    __device__ __forceinline__ Out4(const OutDesc& o, const float* bias, const float* residual, int m0_, int mrows,
+                                    int pos_, int M_, int N_, int seg4_)
+        : od(o), rb(make_rsrc(bias, bias ? (long long)N_ * 4 : 0)),
+          rr(make_rsrc(residual + (residual ? (size_t)m0_ * N_ : 0), residual ? (long long)mrows * N_ * 4 : 0)),
+          m0(m0_), pos(pos_), M(M_), N(N_), flat(o.nseg == 1 && o.rows_per_seq >= (1 << 30)), seg4(seg4_ != 0) {}
+    __device__ __forceinline__ f4u bias(int n) const {
+        return __builtin_bit_cast(f4u, __builtin_amdgcn_raw_buffer_load_b128(rb, n * 4, 0, 0));
+    }
+    __device__ __forceinline__ f4u res(int m, int n) const {
+        return __builtin_bit_cast(f4u, __builtin_amdgcn_raw_buffer_load_b128(rr, ((m - m0) * N + n) * 4, 0, 0));
+    }
+    __device__ __forceinline__ f4u value(const floatx4& acc, const f4u& b, const f4u& r, int epilogue) const {
+        f4u o = {acc[0] + b[0], acc[1] + b[1], acc[2] + b[2], acc[3] + b[3]};
+        if (epilogue == GORCH_HIP_EPI_GELU)
+#pragma unroll
+            for (int v = 0; v < 4; v++) o[v] = gelu_fast(o[v]);
+        return r + o;
+    }
+    __device__ __forceinline__ void put(int m, int n, const f4u& s) const {
+        if (m >= M || n >= N) return;
+        float* p;
+        if (flat) p = od.ptr[0] + (long long)(m + (od.use_pos[0] ? pos : 0)) * od.row_stride[0] + n;
+        else p = od.row(od.col(n, pos), m);
+        if (n + 3 < N && (flat || seg4)) {
+            *reinterpret_cast<f4u*>(p) = s;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (n + v < N) *od.at_p(m, n + v, pos) = s[v];
+        }
+    }
+};
+
+// The tile of this block when each XCD takes one contiguous run of the tiles
+// (blocks are dealt to the 8 XCDs round-robin), walked in bands of `band`
+// tile rows: the tiles in flight on an XCD then share their A and W panels in
+// its L2.
+__device__ __forceinline__ void xcd_tile(int band, int& tx, int& ty) {
+    const int gx = gridDim.x, gy = gridDim.y, L = blockIdx.y * gx + blockIdx.x;
+    const int items = gx * gy, q8 = items >> 3, rem8 = items & 7, xcd = L & 7;
+    const int item = xcd * q8 + min(xcd, rem8) + (L >> 3);
+    const int b = item / (band * gx), t = item - b * band * gx;
+    const int bh = min(band, gy - b * band);
+    ty = b * band + t % bh;
+    tx = t / bh;
+}
+
+// Linear for few tiles (short prompts, narrow weights): the block's G waves
+// share a BM x BN tile of the output and split K: wave w takes the 32-wide
+// steps w, w + G, ... through NST LDS stages of its own. Nothing is shared
+// until the end, so there is no barrier in the loop: a wave waits for its own
+// oldest stage (vmcnt), reads its fragments, and sends the next step's loads
+// into the stage it has just read, with NST - 1 steps in flight behind it
+// (up to 96 KB per CU). The waves' partial tiles meet in LDS and are added
+// in wave order. Products are formed as (W fragment) x (A fragment), which
+// leaves each lane 4 consecutive columns of one row.
+template <int BM, int BN, int G, int NST, bool SPLIT, bool KT>
+__global__ __launch_bounds__(64 * G) void k_gemm_kw(const float* __restrict__ A, const uint16_t* __restrict__ W,
+                                                    const float* __restrict__ bias, const float* residual, OutDesc od,
+                                                    int M, int N, int K, int epilogue, int seg4) {
+    constexpr int TM = BM / 16, TN = BN / 16;
+    constexpr int kA = BM * 128, kStage = kA + BN * 64;   // bytes of one wave's stage
+    constexpr int kLoads = BM / 8 + BN / 16;
+    static_assert(NST == 2 || NST == 3, "stages");
+    static_assert((NST - 1) * kLoads < 64, "vmcnt range");
+    // one array per stage: reads of one do not wait for loads into another
+    __shared__ __align__(16) char st0[G * kStage];
+    __shared__ __align__(16) char st1[G * kStage];
+    __shared__ __align__(16) char st2[NST > 2 ? G * kStage : 16];
+    constexpr int kRed = G * BM * BN * 4;
+    static_assert(kRed <= G * kStage * 2, "partial tiles");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int mrows = min(BM, M - m0), ncols = min(BN, N - n0);
+    const __amdgpu_buffer_rsrc_t rsa = make_rsrc(A + (size_t)m0 * K, (long long)mrows * K * 4);
+    const __amdgpu_buffer_rsrc_t rsw = make_rsrc(W + (size_t)n0 * K, (long long)ncols * K * 2);
+    const int pos = __builtin_amdgcn_readfirstlane(od.pos_dev ? *od.pos_dev : 0);
+
+    floatx4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int nk = (K + kStK - 1) / kStK;
+    const StageLane<8> la(lane, K * 4);
+    const StageLane<4> lw(lane, K * 2);
+    // chunks of the last step that lie past K
+    const int ta = KT && 4 * la.chunk >= K - (nk - 1) * kStK ? kOutOfRange : 0;
+    const int tw = KT && 8 * lw.chunk >= K - (nk - 1) * kStK ? kOutOfRange : 0;
+    const int wofs = wave * kStage;
+    auto issue = [&](char* st, int s) {
+        const bool last = KT && s == nk - 1;
+        la.issue<BM, KT>(st + wofs, rsa, K * 4, s < nk ? s * 128 : kOutOfRange, last ? ta : 0);
+        lw.issue<BN, KT>(st + wofs + kA, rsw, K * 2, s < nk ? s * 64 : kOutOfRange, last ? tw : 0);
+    };
+    struct Frags {
+        float4 a[TM][2];
+        bf16x8 w[TN];
+    };
+    const int ra0 = wofs + r * 128 + 16 * ((2 * g) ^ (r & 7)), ra1 = wofs + r * 128 + 16 * ((2 * g + 1) ^ (r & 7));
+    const int rw0 = wofs + kA + r * 64 + 16 * (g ^ ((r >> 1) & 3));
+    auto read = [&](const char* st, Frags& f) {
+#pragma unroll
+        for (int j = 0; j < TN; j++) f.w[j] = *reinterpret_cast<const bf16x8*>(st + (rw0 + j * 1024));
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            f.a[i][0] = *reinterpret_cast<const float4*>(st + (ra0 + i * 2048));
+            f.a[i][1] = *reinterpret_cast<const float4*>(st + (ra1 + i * 2048));
+        }
+    };
+    auto mul = [&](const Frags& f) {
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            bf16x8 hi, lo;
+            a_terms<SPLIT>(f.a[i][0], f.a[i][1], hi, lo);
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] = mfma16x16x32(f.w[j], hi, acc[i][j]);
+            if constexpr (SPLIT)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] = mfma16x16x32(f.w[j], lo, acc[i][j]);
+        }
+    };
+    // steps of this wave; the last rounds' missing ones read zeros
+    const int rounds = (nk + G - 1) / G;
+    issue(st0, wave);
+    issue(st1, wave + G);
+    if constexpr (NST > 2) issue(st2, wave + 2 * G);
+    // one round: wait for the stage (its loads are the oldest NST - 1 stages
+    // are newer), read it, refill it, multiply
+    constexpr int kWait = (NST - 1) * kLoads;
+    auto round = [&](char* st, int it) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt((kWait & 15) | (7 << 4) | (15 << 8) | ((kWait >> 4) << 14));
+        asm volatile("" ::: "memory");
+        Frags f;
+        read(st, f);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the stage has been read
+        asm volatile("" ::: "memory");
+        issue(st, wave + (it + NST) * G);
+        mul(f);
+    };
+    int it = 0;
+    for (; it + NST <= rounds; it += NST) {
+        round(st0, it);
+        round(st1, it + 1);
+        if constexpr (NST > 2) round(st2, it + 2);
+    }
+    if (it < rounds) round(st0, it);
+    if constexpr (NST > 2)
+        if (it + 1 < rounds) round(st1, it + 1);
+    // every load has landed before the stages hold the partial tiles
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    float4* p0 = reinterpret_cast<float4*>(st0);
+    float4* p1 = reinterpret_cast<float4*>(st1);
+    auto part = [&](int w, int f) -> float4* { return (w < G / 2 ? p0 + w * TM * TN * 64 : p1 + (w - G / 2) * TM * TN * 64) + f * 64 + lane; };
+    static_assert((G / 2) * TM * TN * 1024 <= G * kStage, "partial tiles fit a stage");
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            *part(wave, i * TN + j) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+    __syncthreads();
+    const Out4 out(od, bias, residual, m0, mrows, pos, M, N, seg4);
+#pragma unroll
+    for (int f0 = 0; f0 < TM * TN; f0 += G) {
+        const int f = f0 + wave;
+        if (TM * TN % G != 0 && f >= TM * TN) break;
+        const int m = m0 + (f / TN) * 16 + r, n = n0 + (f % TN) * 16 + 4 * g;
+        const Out4::f4u bv = out.bias(n), rv = out.res(m, n);
+        floatx4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < G; w++) {
+            const float4 v = *part(w, f);
+            s = floatx4{s[0] + v.x, s[1] + v.y, s[2] + v.z, s[3] + v.w};
+        }
+        out.put(m, n, out.value(s, bv, rv, epilogue));
+    }
+}
+
+// Linear for many tiles (long prompts): 8 waves share a 256 x (32 TN) tile,
+// each a 64 x (16 TN) part of it, through three LDS stages.
+//
+// Two waves run on each SIMD, half a step apart: while waves 0-3 multiply a
+// stage (registers only), waves 4-7 read its fragments and send the loads of
+// the stage after next, and the other way round in the next half step, so
+// the matrix cores wait neither for the fragment reads nor for the barrier.
+// 4096^3 runs at 583 TFLOP/s (1,165 on the matrix cores, two terms; this
+// card's library bf16 product of that size 1,150-1,240): what is left is the
+// loads' share of L2 and LDS (with the loads off 178 us, only the loads 128,
+// together 236).
+// A wave waits for its own loads (vmcnt, all but the newest stage) before the
+// barrier behind which the next stage is first read.
+template <int TN, bool SPLIT, bool KT>
+__global__ __launch_bounds__(512, 2) void k_gemm_pp(const float* __restrict__ A, const uint16_t* __restrict__ W,
+                                                    const float* __restrict__ bias, const float* residual, OutDesc od,
+                                                    int M, int N, int K, int epilogue, int seg4, int band) {
+    constexpr int TM = 4, BM = 256, BN = 32 * TN, NW = 8;
+    constexpr int LA = BM / 8 / NW, LW = (BN / 16 + NW - 1) / NW;  // loads per wave and stage
+    constexpr int kA = BM * 128, kStage = kA + LW * NW * 1024;     // bytes (W groups past BN: zeros, unread)
+    __shared__ __align__(16) char st0[kStage];
+    __shared__ __align__(16) char st1[kStage];
+    __shared__ __align__(16) char st2[kStage];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave & 3, wn = wave >> 2, r = lane & 15, g = lane >> 4;
+    int tx = blockIdx.x, ty = blockIdx.y;
+    if (band) xcd_tile(band, tx, ty);
+    const int m0 = ty * BM, n0 = tx * BN;
+    const int mrows = min(BM, M - m0), ncols = min(BN, N - n0);
+    const __amdgpu_buffer_rsrc_t rsa = make_rsrc(A + (size_t)m0 * K, (long long)mrows * K * 4);
+    const __amdgpu_buffer_rsrc_t rsw = make_rsrc(W + (size_t)n0 * K, (long long)ncols * K * 2);
+    const int pos = __builtin_amdgcn_readfirstlane(od.pos_dev ? *od.pos_dev : 0);
+
+    floatx4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    const int nk = (K + kStK - 1) / kStK;
+    const StageLane<8> la(lane, K * 4);
+    const StageLane<4> lw(lane, K * 2);
+    const int ta = KT && 4 * la.chunk >= K - (nk - 1) * kStK ? kOutOfRange : 0;
+    const int tw = KT && 8 * lw.chunk >= K - (nk - 1) * kStK ? kOutOfRange : 0;
+    const int awave = wave * LA * 8 * K * 4, wwave = wave * LW * 16 * K * 2;
+    auto issue = [&](char* st, int s) {
+        const bool last = KT && s == nk - 1;
+        la.issue<LA * 8, KT>(st + wave * LA * 1024, rsa, K * 4, s < nk ? s * 128 + awave : kOutOfRange, last ? ta : 0);
+        lw.issue<LW * 16, KT>(st + kA + wave * LW * 1024, rsw, K * 2, s < nk ? s * 64 + wwave : kOutOfRange,
+                              last ? tw : 0);
+    };
+    const int ra0 = wm * 8192 + r * 128 + 16 * ((2 * g) ^ (r & 7)), ra1 = wm * 8192 + r * 128 + 16 * ((2 * g + 1) ^ (r & 7));
+    const int rw0 = kA + wn * TN * 1024 + r * 64 + 16 * (g ^ ((r >> 1) & 3));
+    bf16x8 fw[TN];
+    float4 fa[TM][2];
+    auto read = [&](const char* st) {
+#pragma unroll
+        for (int j = 0; j < TN; j++) fw[j] = *reinterpret_cast<const bf16x8*>(st + (rw0 + j * 1024));
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            fa[i][0] = *reinterpret_cast<const float4*>(st + (ra0 + i * 2048));
+            fa[i][1] = *reinterpret_cast<const float4*>(st + (ra1 + i * 2048));
+        }
+    };
+    auto mul = [&] {
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            bf16x8 hi, lo;
+            a_terms<SPLIT>(fa[i][0], fa[i][1], hi, lo);
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] = mfma16x16x32(fw[j], hi, acc[i][j]);
+            if constexpr (SPLIT)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] = mfma16x16x32(fw[j], lo, acc[i][j]);
+        }
+    };
+    constexpr int kWait = LA + LW;  // the newest stage's loads may stay in flight
+    constexpr int kVm = (kWait & 15) | (7 << 4) | (15 << 8) | ((kWait >> 4) << 14), kVmLgkm = kVm & ~(15 << 8);
+    constexpr int kLgkm = 0xc07f;
+    auto meet = [&](auto wait) {
+        asm volatile("" ::: "memory");
+        if constexpr (decltype(wait)::value != 0) __builtin_amdgcn_s_waitcnt(decltype(wait)::value);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+    };
+    using C0 = std::integral_constant<int, 0>;
+    using CVm = std::integral_constant<int, kVm>;
+    using CLgkm = std::integral_constant<int, kLgkm>;
+    using CVmLgkm = std::integral_constant<int, kVmLgkm>;
+    issue(st0, 0);
+    issue(st1, 1);
+    meet(CVm{});
+    auto run = [&](auto late_tag) {
+        constexpr bool LATE = decltype(late_tag)::value;
+        auto step = [&](const char* cur, char* nxt, int s) {
+            read(cur);
+            issue(nxt, s + 2);
+            if constexpr (LATE) meet(CVmLgkm{});
+            else meet(CLgkm{});
+            __builtin_amdgcn_s_setprio(1);
+            mul();
+            __builtin_amdgcn_s_setprio(0);
+            if constexpr (LATE) meet(C0{});
+            else meet(CVm{});
+        };
+        if constexpr (LATE) meet(C0{});
+        int s = 0;
+        for (; s + 3 <= nk; s += 3) {
+            step(st0, st2, s);
+            step(st1, st0, s + 1);
+            step(st2, st1, s + 2);
+        }
+        if (s < nk) step(st0, st2, s);
+        if (s + 1 < nk) step(st1, st0, s + 1);
+        if constexpr (!LATE) meet(C0{});
+    };
+    if (wave < 4) run(std::false_type{});
+    else run(std::true_type{});
+    const Out4 out(od, bias, residual, m0, mrows, pos, M, N, seg4);
+    const int nw = n0 + wn * TN * 16 + 4 * g, mw = m0 + wm * 64 + r;
+    Out4::f4u bv[TN], rv[2][TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        bv[j] = out.bias(nw + 16 * j);
+        rv[0][j] = out.res(mw, nw + 16 * j);
+    }
+    // the next 16 rows' residual is requested before this one's stores (a
+    // load after a store would wait for the store's write)
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        if (i + 1 < TM)
+#pragma unroll
+            for (int j = 0; j < TN; j++) rv[(i + 1) & 1][j] = out.res(mw + 16 * (i + 1), nw + 16 * j);
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            out.put(mw + 16 * i, nw + 16 * j, out.value(acc[i][j], bv[j], rv[i & 1][j], epilogue));
+    }
+}
+
+// every output segment starts at a multiple of 4 columns
+static int segments_by_4(const OutDesc& od) {
+    int ok = 1;
+    for (int i = 0; i + 1 < od.nseg; i++) ok &= od.n_end[i] % 4 == 0;
+    return ok;
+}
+
+template <int TN>
+static void launch_pp(hipStream_t s, const float* A, const uint16_t* W, const float* bias, const float* residual,
+                      const OutDesc& od, int M, int N, int K, int epilogue, bool act_bf16) {
+    const dim3 grid((N + 32 * TN - 1) / (32 * TN), (M + 255) / 256);
+    const int seg4 = segments_by_4(od);
+    // bands of 4 tile rows per XCD: 8192 x 1600 x 6400 347 -> 328 us (8: 333)
+    constexpr int band = 4;
+#define GH_PP(SP, KTV)                                                                                         \
+    hipLaunchKernelGGL((k_gemm_pp<TN, SP, KTV>), grid, dim3(512), 0, s, A, W, bias, residual, od, M, N, K, epilogue, \
+                       seg4, band)
+    if (K % kStK) {
+        if (act_bf16) GH_PP(false, true);
+        else GH_PP(true, true);
+    } else {
+        if (act_bf16) GH_PP(false, false);
+        else GH_PP(true, false);
+    }
+#undef GH_PP
+}
+
+template <int BM, int BN, int G, int NST>
+static void launch_kw(hipStream_t s, const float* A, const uint16_t* W, const float* bias, const float* residual,
+                      const OutDesc& od, int M, int N, int K, int epilogue, bool act_bf16) {
+    const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+    const int seg4 = segments_by_4(od);
+#define GH_KW(SP, KTV)                                                                                            \
+    hipLaunchKernelGGL((k_gemm_kw<BM, BN, G, NST, SP, KTV>), grid, dim3(64 * G), 0, s, A, W, bias, residual, od, M, N, K, \
+                       epilogue, seg4)
+    if (K % kStK) {
+        if (act_bf16) GH_KW(false, true);
+        else GH_KW(true, true);
+    } else {
+        if (act_bf16) GH_KW(false, false);
+        else GH_KW(true, false);
+    }
+#undef GH_KW
+}
+
 // Tile width for k_gemm_db: the most 64-row blocks that still fit one
 // round on the chip (measured at 512 x 768: N = 2304 on 64 x 96, 192
 // blocks, 7.1 us; N = 3072 on 64 x 96, 256 blocks, 7.4 us, against 7.5 /
@@ -493,36 +760,68 @@ static void launch_db(hipStream_t s, const float* A, const uint16_t* W, const fl
     }
 }
 
-template <int BM, int BN, bool SPLIT>
-static void launch_gemm_t(hipStream_t s, const float* A, const uint16_t* W, const float* bias,
-                          const float* residual, const OutDesc& od, int M, int N, int K, int epilogue) {
-    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-    // one register stage for 128 x 128 tiles (more stages cost occupancy:
-    // 4096^3 247 vs 301 us); no K tail: loads with no bound on k (a select
-    // on every offset compiles to branches around the loads)
-    constexpr int pf = 1;
-    if (K % kBK != 0)
-        hipLaunchKernelGGL((k_gemm_bf16w<BM, BN, SPLIT, pf, true>), grid, dim3(256), 0, s, A, W, bias, residual, od, M,
-                           N, K, epilogue);
-    else
-        hipLaunchKernelGGL((k_gemm_bf16w<BM, BN, SPLIT, pf, false>), grid, dim3(256), 0, s, A, W, bias, residual, od,
-                           M, N, K, epilogue);
+// Kernel and tile by estimated time (us), each estimate fitted to measured
+// launches on 256 CUs with the weight beyond L2:
+//   k_gemm_db (64 rows x 32 w columns): 2.5 + steps of 64 x {0.56, 0.78, 0.83}
+//     (w = 2, 3, 4) x blocks / 256. 777 x 1024 x 4096 22.8 (estimate 24),
+//     777 x 1024 x 6144 32.4 (35), 8192 x 1600 x 1600 128 (138).
+//   k_gemm_kw (BM x BN, one block per CU): 1.5 + rounds x (3.5 + K (4 BM +
+//     2 BN) bytes at 75 B/ns), and at least 3.5 + all blocks' bytes at 13.5
+//     TB/s. 97 x 3072 x 768 7.8 on 16 x 32 tiles against 26.8 (db); 32 x 3072
+//     x 768 8.1 / 26.4; 777 x 3072 x 1024 22.5 on 64 x 64 / 29.1.
+//   k_gemm_pp (256 x 32 TN): 3 + rounds x max(steps of 32 x c(TN), the stores
+//     of one tile per CU, 1.86 TN). 8192 x 1600 x 6400 328 at TN = 7 (4 rounds; 348 at 8, 344 at 5)
+//     against 429 for the 128 x 128 tiles without a pipeline it replaced;
+//     2007 x 1600 x 4800 72 / 107 (db 95); 200 x 1600 x 50257 84 / 128.
+enum GemmKind { kDb, kKw16x32, kKw32x32, kKw32x64, kKw64x64, kPp4, kPp5, kPp6, kPp7, kPp8 };
+static GemmKind gemm_kind(int M, int N, int K) {
+    auto cdiv = [](long long a, long long b) { return (a + b - 1) / b; };
+    constexpr double kCus = 256.0;
+    const int w = db_waves(M, N);
+    const double cdb[3] = {0.56, 0.78, 0.83};
+    GemmKind best = kDb;
+    double t = 2.5 + cdiv(K, 64) * cdb[w - 2] * std::max(1.0, cdiv(M, 64) * cdiv(N, 32 * w) / kCus);
+    auto take = [&](GemmKind k, double c) {
+        if (c < t) {
+            t = c;
+            best = k;
+        }
+    };
+    const int kw[4][2] = {{16, 32}, {32, 32}, {32, 64}, {64, 64}};
+    for (int i = 0; i < 4; i++) {
+        const double blocks = (double)cdiv(M, kw[i][0]) * cdiv(N, kw[i][1]);
+        const double bytes = (double)K * (4 * kw[i][0] + 2 * kw[i][1]);
+        take((GemmKind)(kKw16x32 + i),
+             std::max(1.5 + std::ceil(blocks / kCus) * (3.5 + bytes / 75e3), 3.5 + blocks * bytes / 13.5e6));
+    }
+    const double cpp[5] = {1.05, 1.3, 1.43, 1.62, 1.8};
+    for (int tn = 4; tn <= 8; tn++) {
+        const double rounds = std::ceil((double)cdiv(M, 256) * cdiv(N, 32 * tn) / kCus);
+        take((GemmKind)(kPp4 + tn - 4), 3.0 + rounds * std::max(cdiv(K, 32) * cpp[tn - 4], 1.86 * tn));
+    }
+    return best;
 }
 
-// Tile choice: 128 x 128 tiles (k_gemm_bf16w) when they give every CU a
-// block, else the double-buffered 64-row kernel (k_gemm_db).
 int launch_gemm_bf16w(hipStream_t s, const float* A, const uint16_t* W, const float* bias,
                       const float* residual, const OutDesc& od, int M, int N, int K, int epilogue,
                       bool act_bf16) {
-    const long long big = (long long)((M + 127) / 128) * ((N + 127) / 128);
-    if (big < 256) {
-        if (act_bf16) launch_db<false>(s, A, W, bias, residual, od, M, N, K, epilogue);
-        else launch_db<true>(s, A, W, bias, residual, od, M, N, K, epilogue);
-    } else if (act_bf16) {
-        launch_gemm_t<128, 128, false>(s, A, W, bias, residual, od, M, N, K, epilogue);
-    } else {
-        launch_gemm_t<128, 128, true>(s, A, W, bias, residual, od, M, N, K, epilogue);
+#define GH_ARGS s, A, W, bias, residual, od, M, N, K, epilogue
+    switch (gemm_kind(M, N, K)) {
+        case kKw16x32: launch_kw<16, 32, 8, 3>(GH_ARGS, act_bf16); break;
+        case kKw32x32: launch_kw<32, 32, 8, 3>(GH_ARGS, act_bf16); break;
+        case kKw32x64: launch_kw<32, 64, 4, 3>(GH_ARGS, act_bf16); break;
+        case kKw64x64: launch_kw<64, 64, 4, 2>(GH_ARGS, act_bf16); break;
+        case kPp4: launch_pp<4>(GH_ARGS, act_bf16); break;
+        case kPp5: launch_pp<5>(GH_ARGS, act_bf16); break;
+        case kPp6: launch_pp<6>(GH_ARGS, act_bf16); break;
+        case kPp7: launch_pp<7>(GH_ARGS, act_bf16); break;
+        case kPp8: launch_pp<8>(GH_ARGS, act_bf16); break;
+        default:
+            if (act_bf16) launch_db<false>(GH_ARGS);
+            else launch_db<true>(GH_ARGS);
+            break;
     }
+#undef GH_ARGS
     count(CNT_GEMM);
     return check_launch("gemm_bf16w");
 }
