@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "stage_lds.h"
 
 namespace gh {
 
@@ -264,44 +265,11 @@ __global__ __launch_bounds__(128 * WGN) void k_gemm_db(const float* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// Stages loaded straight to LDS (raw buffer loads to LDS, 16 bytes a lane).
-//
-// A stage is BK = 32 wide: A rows stay f32 (128 bytes, 8 chunks of 16) and
-// are split into their bf16 terms as a fragment is read (f32 and hi + lo take
-// the same LDS), W rows are bf16 (64 bytes, 4 chunks). Chunk c of A row i
-// sits at c ^ (i & 7), of W row i at c ^ ((i >> 1) & 3): conflict-free
-// 16-byte fragment reads. Rows past the tile's edge are clamped into it and
-// chunks past K read as zeros (an out-of-range offset), so steps past the
-// last one cost no traffic.
+// k_gemm_kw and k_gemm_pp stage 32-wide steps (stage_lds.h): A rows stay f32
+// (128 bytes, 8 chunks) and are split into their bf16 terms as a fragment is
+// read (f32 and hi + lo take the same LDS), W rows are bf16 (64 bytes, 4
+// chunks).
 constexpr int kStK = 32;
-
-// Lane l of a load takes row l / CH of its group of 64 / CH rows and the
-// chunk that belongs at position l % CH of that row; `chunk` is the same for
-// every group, so a lane's offset is a constant plus a scalar (group row,
-// step). Everything goes through the checked offset: rows past the resource
-// and a step past the last one (kbyte = kOutOfRange) read as zeros, and so do
-// chunks past K when `tail` is kOutOfRange for the lane (0 otherwise).
-template <int CH>
-struct StageLane {
-    int chunk, off;
-    __device__ __forceinline__ StageLane(int lane, int ld) {
-        const int row = lane / CH;
-        chunk = (lane % CH) ^ (CH == 8 ? row : ((row >> 1) & 3));
-        off = row * ld + 16 * chunk;
-    }
-    // copies ROWS rows (stride ld bytes) of the step at byte kbyte to LDS
-    template <int ROWS, bool KT>
-    __device__ __forceinline__ void issue(char* lds, __amdgpu_buffer_rsrc_t rs, int ld, int kbyte, int tail) const {
-        constexpr int RPI = 64 / CH;
-#pragma unroll
-        for (int i = 0; i < ROWS / RPI; i++) {
-            unsigned o = (unsigned)off + (unsigned)(i * RPI * ld + kbyte);
-            if constexpr (KT) o = max(o, (unsigned)tail);
-            typedef __attribute__((address_space(3))) void* lds_ptr;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)(lds + i * 1024), 16, (int)o, 0, 0, 0);
-        }
-    }
-};
 
 // the bf16 terms of 8 consecutive f32 of an A row: hi (truncated) and lo
 // (the remainder rounded), or one rounded term
@@ -469,12 +437,12 @@ __global__ __launch_bounds__(64 * G) void k_gemm_kw(const float* __restrict__ A,
     constexpr int kWait = (NST - 1) * kLoads;
     auto round = [&](char* st, int it) {
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt((kWait & 15) | (7 << 4) | (15 << 8) | ((kWait >> 4) << 14));
+        __builtin_amdgcn_s_waitcnt(wait_vm(kWait, false));
         asm volatile("" ::: "memory");
         Frags f;
         read(st, f);
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the stage has been read
+        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);  // the stage has been read
         asm volatile("" ::: "memory");
         issue(st, wave + (it + NST) * G);
         mul(f);
@@ -595,8 +563,6 @@ __global__ __launch_bounds__(512, 2) void k_gemm_pp(const float* __restrict__ A,
         }
     };
     constexpr int kWait = LA + LW;  // the newest stage's loads may stay in flight
-    constexpr int kVm = (kWait & 15) | (7 << 4) | (15 << 8) | ((kWait >> 4) << 14), kVmLgkm = kVm & ~(15 << 8);
-    constexpr int kLgkm = 0xc07f;
     auto meet = [&](auto wait) {
         asm volatile("" ::: "memory");
         if constexpr (decltype(wait)::value != 0) __builtin_amdgcn_s_waitcnt(decltype(wait)::value);
@@ -606,9 +572,9 @@ __global__ __launch_bounds__(512, 2) void k_gemm_pp(const float* __restrict__ A,
         asm volatile("" ::: "memory");
     };
     using C0 = std::integral_constant<int, 0>;
-    using CVm = std::integral_constant<int, kVm>;
-    using CLgkm = std::integral_constant<int, kLgkm>;
-    using CVmLgkm = std::integral_constant<int, kVmLgkm>;
+    using CVm = std::integral_constant<int, wait_vm(kWait, false)>;
+    using CLgkm = std::integral_constant<int, kWaitLgkm0>;
+    using CVmLgkm = std::integral_constant<int, wait_vm(kWait, true)>;
     issue(st0, 0);
     issue(st1, 1);
     meet(CVm{});

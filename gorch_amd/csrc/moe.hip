@@ -22,6 +22,7 @@
 
 #include "common.h"
 #include "gemm_wide.h"
+#include "stage_lds.h"
 
 namespace gh {
 
@@ -605,6 +606,178 @@ static int launch_moe_wide(hipStream_t s, dim3 grid, const uint16_t* Ahi, const 
                                                            cslice, xcd_map, ws);
 }
 
+// Grouped expert GEMM for few rows per expert (a decode batch, a short
+// prompt): the wide tiles give such a layer only E x N / 256 blocks, each
+// streaming its weight panel alone (the down GEMM of 16 tokens: 32 blocks, 45
+// us for 67 MB). Here a block takes BM rows x BN columns (DUAL: of gate and up
+// each) and its G waves split K: wave w takes the 64-wide steps w, w + G, ...
+// through NST LDS stages of its own, waiting only for its own oldest stage;
+// the waves' partial tiles are added in LDS in wave order. blockIdx.x: column
+// tile, y: row tile of the table, z: BM-row chunk of that tile.
+template <bool DUAL, int BM, int BN, int G, int NST>
+__global__ __launch_bounds__(64 * G) void k_moe_kw(const uint16_t* __restrict__ Ahi, const uint16_t* __restrict__ Alo,
+                                                   const uint16_t* __restrict__ W1, const uint16_t* __restrict__ W2,
+                                                   const float* __restrict__ b1, const float* __restrict__ b2,
+                                                   float* __restrict__ C, uint16_t* __restrict__ Chi,
+                                                   uint16_t* __restrict__ Clo, int N, int Kd, MoeWs ws) {
+    constexpr int TM = BM / 16, TN = BN / 16, NB = DUAL ? 2 : 1;
+    constexpr int kA = BM * 128, kW = BN * 128, kStage = 2 * kA + NB * kW;  // bytes of a wave's stage
+    constexpr int kLoads = kStage / 1024;
+    static_assert(NST == 2 || NST == 3, "stages");
+    static_assert((NST - 1) * kLoads < 64, "vmcnt range");
+    __shared__ __align__(16) char st0[G * kStage];
+    __shared__ __align__(16) char st1[G * kStage];
+    __shared__ __align__(16) char st2[NST > 2 ? G * kStage : 16];
+    constexpr int NF = NB * TM * TN;  // 16 x 16 partial tiles per wave
+    static_assert((G / 2) * NF * 1024 <= G * kStage, "partial tiles fit a stage");
+    const int ty = blockIdx.y;
+    if (ty >= *ws.ntiles) return;
+    const int e = ws.tile_e[ty], row0 = blockIdx.z * BM;
+    const int nrows = min(BM, ws.tile_n[ty] - row0);
+    if (nrows <= 0) return;
+    const int r0 = __builtin_amdgcn_readfirstlane(ws.tile_r0[ty] + row0), n0 = blockIdx.x * BN;
+    const int ncols = min(BN, N - n0);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const size_t wofs = ((size_t)__builtin_amdgcn_readfirstlane(e) * N + n0) * Kd;
+    const __amdgpu_buffer_rsrc_t rh = make_rsrc(Ahi + (size_t)r0 * Kd, (long long)nrows * Kd * 2);
+    const __amdgpu_buffer_rsrc_t rl = make_rsrc(Alo + (size_t)r0 * Kd, (long long)nrows * Kd * 2);
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(W1 + wofs, (long long)ncols * Kd * 2);
+    const __amdgpu_buffer_rsrc_t rw2 = make_rsrc(W2 + (DUAL ? wofs : 0), DUAL ? (long long)ncols * Kd * 2 : 0);
+
+    floatx4 acc[NB][TM][TN];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[b][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int nk = (Kd + 63) / 64, rounds = (nk + G - 1) / G;
+    const StageLane<8> ln(lane, Kd * 2);
+    const int tail = 8 * ln.chunk >= Kd - (nk - 1) * 64 ? kOutOfRange : 0;
+    const int mine = wave * kStage;
+    auto issue = [&](char* st, int s) {
+        const int kb = s < nk ? s * 128 : kOutOfRange, t = s == nk - 1 ? tail : 0;
+        ln.issue<BM, true>(st + mine, rh, Kd * 2, kb, t);
+        ln.issue<BM, true>(st + (mine + kA), rl, Kd * 2, kb, t);
+        ln.issue<BN, true>(st + (mine + 2 * kA), rw, Kd * 2, kb, t);
+        if constexpr (DUAL) ln.issue<BN, true>(st + (mine + 2 * kA + kW), rw2, Kd * 2, kb, t);
+    };
+    const int f0 = mine + r * 128 + 16 * (g ^ (r & 7)), f1 = mine + r * 128 + 16 * ((4 + g) ^ (r & 7));
+    struct Frags {
+        bf16x8 a[2][2][TM], w[2][NB][TN];  // [half of the step][plane / weight]
+    };
+    auto read = [&](const char* st, Frags& f) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int o = h ? f1 : f0;
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+#pragma unroll
+                for (int i = 0; i < TM; i++) f.a[h][q][i] = *reinterpret_cast<const bf16x8*>(st + (o + q * kA + i * 2048));
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    f.w[h][b][j] = *reinterpret_cast<const bf16x8*>(st + (o + 2 * kA + b * kW + j * 2048));
+        }
+    };
+    auto mul = [&](const Frags& f) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+#pragma unroll
+                        for (int j = 0; j < TN; j++)
+                            acc[b][i][j] = mfma16x16x32(f.w[h][b][j], f.a[h][q][i], acc[b][i][j]);
+    };
+    issue(st0, wave);
+    issue(st1, wave + G);
+    if constexpr (NST > 2) issue(st2, wave + 2 * G);
+    auto round = [&](char* st, int it) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(wait_vm((NST - 1) * kLoads, false));
+        asm volatile("" ::: "memory");
+        Frags f;
+        read(st, f);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);  // the stage has been read
+        asm volatile("" ::: "memory");
+        issue(st, wave + (it + NST) * G);
+        mul(f);
+    };
+    int it = 0;
+    for (; it + NST <= rounds; it += NST) {
+        round(st0, it);
+        round(st1, it + 1);
+        if constexpr (NST > 2) round(st2, it + 2);
+    }
+    if (it < rounds) round(st0, it);
+    if constexpr (NST > 2)
+        if (it + 1 < rounds) round(st1, it + 1);
+    // every load has landed before the stages hold the partial tiles
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    float4* p0 = reinterpret_cast<float4*>(st0);
+    float4* p1 = reinterpret_cast<float4*>(st1);
+    auto part = [&](int w, int f) -> float4* {
+        return (w < G / 2 ? p0 + w * NF * 64 : p1 + (w - G / 2) * NF * 64) + f * 64 + lane;
+    };
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const floatx4 v = acc[b][i][j];
+                *part(wave, (b * TM + i) * TN + j) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+    __syncthreads();
+    auto total = [&](int f) {
+        float4 s = *part(0, f);
+#pragma unroll
+        for (int w = 1; w < G; w++) {
+            const float4 v = *part(w, f);
+            s = make_float4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w);
+        }
+        return s;
+    };
+#pragma unroll
+    for (int q0 = 0; q0 < TM * TN; q0 += G) {
+        const int q = q0 + wave;
+        if (TM * TN % G != 0 && q >= TM * TN) break;
+        // lane: row r, columns 4g .. 4g + 3 of the 16 x 16 tile; N % 8 == 0
+        const int row = (q / TN) * 16 + r, col = (q % TN) * 16 + 4 * g;
+        const float4 s = total(q), u = total(DUAL ? TM * TN + q : q);
+        if (row >= nrows || col >= ncols) continue;
+        const size_t o = (size_t)(r0 + row) * N + n0 + col, bo = (size_t)e * N + n0 + col;
+        float v[4] = {s.x, s.y, s.z, s.w};
+        if (b1)
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] += b1[bo + c];
+        if constexpr (DUAL) {
+            float up[4] = {u.x, u.y, u.z, u.w};
+            if (b2)
+#pragma unroll
+                for (int c = 0; c < 4; c++) up[c] += b2[bo + c];
+            uint16_t hi[4], lo[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) split_hi_lo1(v[c] * sigmoidf_ref(v[c]) * up[c], hi[c], lo[c]);
+            *reinterpret_cast<uint2*>(Chi + o) =
+                make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
+            *reinterpret_cast<uint2*>(Clo + o) =
+                make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
+        } else {
+            const float w = ws.perm_w[r0 + row];  // weighted = exOut * w
+            *reinterpret_cast<float4*>(C + o) = make_float4(v[0] * w, v[1] * w, v[2] * w, v[3] * w);
+        }
+    }
+}
+
 }  // namespace gh
 
 using namespace gh;
@@ -677,14 +850,46 @@ extern "C" int gorch_hip_moe_forward(void* stream, const gorch_hip_moe_weights* 
         hipLaunchKernelGGL(k_moe_gather_split<kMaxTopK>, dim3(gblocks), dim3(256), 0, s, x, ws.inv, xhi, xlo, M, K,
                            d);
     GH_TRY(check_launch("moe_gather"));
-    GH_TRY((launch_moe_wide<true, kWideBNDual>(s, dim3((F + kWideBNDual - 1) / kWideBNDual, max_tiles), xhi, xlo,
-                                              w->wgate, w->wup, w->bgate, w->bup, nullptr, hhi, hlo, F, d, 0, ws)));
+    // At most this many row tiles are live: one per expert reached and one
+    // more per 128 rows. Few rows per expert: K split over the waves of small
+    // tiles (k_moe_kw), else the wide tiles. Down GEMM, whole layer in us (1024 x 4096, 8
+    // experts, top-2), wide / kw 16x32 / 32x32 / 32x64: 16 tokens (4 rows an
+    // expert) 103 / 64 / 66 / 68; 64 (16) 107 / 73 / 70 / 73; 128 (32) 110 /
+    // 84 / 76 / 72; 512 (128) 158 / 183 / 152 / 135; 1024 (256) 201 / - / 227
+    // / 217. With few column tiles the wide form stays short of CUs at any
+    // length (1000 tokens, 512 x 1368, 4 experts, 38 blocks: 74 / - / 67 / 61).
+    const int avg = MK / E;
+    const long long live = std::min(E, MK) + MK / tile_rows;
+    auto chunks = [&](int bm) { return (unsigned)((std::min(M, tile_rows) + bm - 1) / bm); };
+    if (live * ((F + kWideBNDual - 1) / kWideBNDual) <= 128 && avg <= 64) {
+        // the wide form would run on half the CUs or fewer (16 tokens, 512 x
+        // 1368, 4 experts: 47 -> 42 us a layer)
+        hipLaunchKernelGGL((k_moe_kw<true, 32, 32, 4, 2>), dim3((F + 31) / 32, max_tiles, chunks(32)), dim3(256), 0, s,
+                           xhi, xlo, w->wgate, w->wup, w->bgate, w->bup, nullptr, hhi, hlo, F, d, ws);
+        GH_TRY(check_launch("moe_kw_gate_up"));
+    } else {
+        GH_TRY((launch_moe_wide<true, kWideBNDual>(s, dim3((F + kWideBNDual - 1) / kWideBNDual, max_tiles), xhi, xlo,
+                                                  w->wgate, w->wup, w->bgate, w->bup, nullptr, hhi, hlo, F, d, 0, ws)));
+    }
     // the down GEMM unsplit over K (one slice of partials in yg)
     const int nsl = 1;
     const long long cslice = (long long)MK * d;
-    GH_TRY((launch_moe_wide<false, kWideBNDown>(s, dim3((d + kWideBNDown - 1) / kWideBNDown, max_tiles, nsl), hhi,
-                                                hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr, d,
-                                                F, cslice, ws)));
+    if (avg <= 192 || live * ((d + kWideBNDown - 1) / kWideBNDown) <= 64) {
+        if (avg <= 8)
+            hipLaunchKernelGGL((k_moe_kw<false, 16, 32, 8, 2>), dim3((d + 31) / 32, max_tiles, chunks(16)), dim3(512), 0, s,
+                               hhi, hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, ws);
+        else if (avg <= 16)
+            hipLaunchKernelGGL((k_moe_kw<false, 32, 32, 4, 3>), dim3((d + 31) / 32, max_tiles, chunks(32)), dim3(256), 0, s,
+                               hhi, hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, ws);
+        else
+            hipLaunchKernelGGL((k_moe_kw<false, 32, 64, 4, 2>), dim3((d + 63) / 64, max_tiles, chunks(32)), dim3(256), 0, s,
+                               hhi, hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, ws);
+        GH_TRY(check_launch("moe_kw_down"));
+    } else {
+        GH_TRY((launch_moe_wide<false, kWideBNDown>(s, dim3((d + kWideBNDown - 1) / kWideBNDown, max_tiles, nsl), hhi,
+                                                    hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr,
+                                                    d, F, cslice, ws)));
+    }
     const int cblocks = (int)std::min<int64_t>(8192, ((int64_t)M * d / 4 + 255) / 256);
     if (K <= 2)
         hipLaunchKernelGGL(k_moe_combine<2>, dim3(cblocks), dim3(256), 0, s, ws.yg, ws.inv, ws.topi, out, M, K, d, nsl,

@@ -1,0 +1,53 @@
+"""The MoE layer with few rows per expert (the K-split expert GEMMs) at the
+edges of their tiles: one row to several 16- and 32-row chunks per expert,
+experts without rows, every token on one expert, column and K remainders.
+
+Bound: float64 from the same bf16 weights, 2e-5 of the output in the 2-norm
+(two bf16 terms per activation through two GEMMs measure 0.9e-5; one term
+would give 3e-3).
+"""
+import numpy as np
+import pytest
+import torch
+
+from gorch_amd import synthetic as syn
+from gorch_amd.bf16 import bf16_to_f32
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(w, x, logits):
+    order = np.argsort(-logits, axis=1, kind="stable")[:, : w["top_k"]]
+    val = np.take_along_axis(logits.astype(np.float64), order, 1)
+    wts = np.exp(val - val.max(1, keepdims=True))
+    wts /= wts.sum(1, keepdims=True)
+    out = np.zeros(x.shape, np.float64)
+    for e in range(w["experts"]):
+        rows, slot = np.nonzero(order == e)
+        if not len(rows):
+            continue
+        W = {k: bf16_to_f32(w[k][e]).astype(np.float64) for k in ("wgate", "wup", "wdown")}
+        xe = x[rows].astype(np.float64)
+        g = xe @ W["wgate"].T + w["bgate"][e]
+        u = xe @ W["wup"].T + w["bup"][e]
+        y = (g / (1 + np.exp(-g)) * u) @ W["wdown"].T + w["bdown"][e]
+        np.add.at(out, rows, y * wts[rows, slot][:, None])
+    return out
+
+
+@pytest.mark.parametrize("M,dim,ffn,E,K,skew", [
+    (1, 64, 64, 4, 1, 0), (1, 72, 104, 8, 2, 0), (16, 264, 520, 8, 2, 0), (16, 64, 2056, 8, 2, 99), (33, 128, 192, 4, 2, 0),
+    (70, 1032, 136, 8, 2, 0), (64, 512, 1368, 4, 2, 0), (150, 96, 264, 4, 2, 99), (300, 200, 328, 4, 2, 0),
+    (129, 64, 4096, 2, 1, 0), (700, 320, 256, 8, 2, 1), (31, 40, 24, 64, 8, 0),
+])
+def test_moe_few_rows(gpu, M, dim, ffn, E, K, skew):
+    """skew pushes tokens towards expert 0 (99: every token's first choice)."""
+    x, logits, w = syn.moe_inputs(M=M, dim=dim, ffn=ffn, experts=E, top_k=K, seed=M + dim)
+    rng = np.random.default_rng(M)
+    logits[:, 0] += skew
+    for k in ("bgate", "bup", "bdown"):
+        w[k] = [(0.1 * rng.standard_normal(b.shape)).astype(np.float32) for b in w[k]]
+    dev = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    out, _, _ = gpu.MoE(w).forward(dev(x), dev(logits))
+    ref = reference(w, x, logits)
+    assert np.linalg.norm(out.cpu().numpy() - ref) <= 2e-5 * np.linalg.norm(ref)
