@@ -165,8 +165,23 @@ def _p(t):
 
 
 def _stream():
+    """The current HIP stream's handle on the current device. The raw query
+    takes 0.1 us where building a torch.cuda.Stream object takes 2.8, more
+    than a small kernel's launch."""
+    torch_c = _torch_c or _load_torch()
+    return torch_c._cuda_getCurrentRawStream(torch_c._cuda_getDevice())
+
+
+_torch_c = None
+
+
+def _load_torch():
+    global _torch_c
     import torch
-    return torch.cuda.current_stream().cuda_stream
+
+    torch.cuda.current_stream()  # initialises the CUDA (HIP) state once
+    _torch_c = torch._C
+    return _torch_c
 
 
 def init(device: int = 0) -> None:
