@@ -399,6 +399,10 @@ bool gemv_m1_prologue_ok(int K);
 // The one-row GEMV can pair the gate and up rows of a [2F, K] weight
 // (LinearExtras::pair_swiglu = F).
 bool gemv_pair_swiglu_ok(int F, int K);
+// The gate/up product of more than 16 rows with SwiGLU in its epilogue
+// (gemm.hip): y [M, N] from x [M, K] and W [2N, K].
+bool gemm_pair_swiglu_ok(int M, int N, int K);
+int launch_gemm_pair_swiglu(hipStream_t s, const float* x, const uint16_t* W, float* y, int M, int N, int K);
 int launch_swiglu(hipStream_t s, const float* g, const float* v, float* y, int64_t n);
 
 // A tensor entry of a safetensors header (safetensors.hip): dtype

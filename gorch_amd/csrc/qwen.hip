@@ -15,8 +15,9 @@
 //   4. RMSNorm_ffn applied as the gate/up GEMV loads x1 (one [2F, d] weight),
 //      gate row j and up row F + j in one wave so it writes silu(gate) * up;
 //   5. down GEMV with the residual add.
-// Longer inputs (prefill) take the same steps with the norms and SwiGLU as
-// launches of their own and the matrix-core GEMM for the Linears.
+// Longer inputs (prefill) take the same steps with the norms as launches of
+// their own and the matrix-core GEMMs for the Linears, SwiGLU in the gate/up
+// GEMM's epilogue.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -86,9 +87,14 @@ static int qwen_block_core(hipStream_t s, const gorch_hip_qwen_block* b, float* 
         return launch_linear_bf16_od(s, gu, b->wdown, nullptr, x1, OutDesc::plain(x, d), 1, d, F,
                                      GORCH_HIP_EPI_NONE, sw);
     }
-    // longer inputs: h = RMSNorm_ffn(x1), gate and up as two column
-    // segments of one GEMM, SwiGLU, down
+    // longer inputs: h = RMSNorm_ffn(x1), the gate/up GEMM with SwiGLU in its
+    // epilogue, down; where that GEMM's tiles split K, gate and up as two
+    // column segments and a SwiGLU launch
     GH_TRY(launch_rmsnorm(s, x1, b->norm_ffn, h, S, d, b->eps));
+    if (gemm_pair_swiglu_ok(S, F, d)) {
+        GH_TRY(launch_gemm_pair_swiglu(s, h, b->wgate_up, gu, S, F, d));
+        return launch_linear_bf16(s, gu, b->wdown, nullptr, x1, x, S, d, F, GORCH_HIP_EPI_NONE);
+    }
     float* gate = gu;
     float* up = gu + (size_t)S * F;
     OutDesc od{};

@@ -157,6 +157,92 @@ __global__ __launch_bounds__(256) void k_norm_rope_rows(const float* x, float* y
     if (lane < nl) *reinterpret_cast<float4*>(y + (size_t)r * hd + 4 * lane) = make_float4(o[0], o[1], o[2], o[3]);
 }
 
+// The same for a prompt: one block per token, its q and k heads dealt to 4
+// waves, NL = hd / 4 lanes a row (64 / NL rows side by side in a wave) and up
+// to 4 rows per lane group. The token's cos / sin are loaded once per wave
+// instead of once per row, every load goes out before the first use, and no
+// lane idles (a row of 128 took half a wave): 777 tokens, 16 + 8 heads of 128
+// 9.6 -> 7.2 us under the profiler. Same operations per row as k_norm_rope_rows, in its order.
+constexpr int kTokRows = 4;
+template <int NL>
+__global__ __launch_bounds__(256) void k_norm_rope_tok(const float* xq, float* yq, int hq,
+                                                       const float* __restrict__ gq, const float* xk, float* yk,
+                                                       int hk, const float* __restrict__ gk, float eps, int start_pos,
+                                                       const float* __restrict__ cosT,
+                                                       const float* __restrict__ sinT, int neox) {
+#pragma clang fp contract(off)
+    constexpr int HD = 4 * NL, half = HD / 2, RPW = 64 / NL;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane % NL, sub = lane / NL;
+    const int tok = blockIdx.x, p = start_pos + tok;
+    const bool lo = c < NL / 2;
+    float4 v[kTokRows];
+    float* out[kTokRows];
+    bool isq[kTokRows];
+#pragma unroll
+    for (int i = 0; i < kTokRows; i++) {
+        // rows past the last head repeat it and are not stored
+        const int h = wave * RPW + sub + i * 4 * RPW, hc = min(h, hq + hk - 1);
+        isq[i] = hc < hq;
+        const size_t o = isq[i] ? ((size_t)tok * hq + hc) * HD : ((size_t)tok * hk + hc - hq) * HD;
+        v[i] = *reinterpret_cast<const float4*>((isq[i] ? xq : xk) + o + 4 * c);
+        out[i] = h < hq + hk ? (isq[i] ? yq : yk) + o + 4 * c : nullptr;
+    }
+    const __amdgpu_buffer_rsrc_t rgq = make_rsrc(gq, gq ? HD * 4 : 0), rgk = make_rsrc(gk, gk ? HD * 4 : 0);
+    const float4 g0 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rgq, 16 * c, 0, 0));
+    const float4 g1 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rgk, 16 * c, 0, 0));
+    float co[4], sn[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int k = 4 * c + q;
+        const int i = neox ? 2 * c + q / 2 : (lo ? k : k - half);
+        co[q] = cosT[(size_t)p * half + i];
+        sn[q] = sinT[(size_t)p * half + i];
+    }
+#pragma unroll
+    for (int i = 0; i < kTokRows; i++) {
+        float4 x = v[i];
+        double s = ((double)x.x * (double)x.x + (double)x.y * (double)x.y) +
+                   ((double)x.z * (double)x.z + (double)x.w * (double)x.w);
+        // the sum over the row's NL lanes
+        s += dpp_d<kDppQuadSwap1>(s);
+        s += dpp_d<kDppQuadSwap2>(s);
+        s += dpp_d<kDppRowHalfMirror>(s);
+        s += dpp_d<kDppRowMirror>(s);
+        if constexpr (NL == 32) {
+            const double a = readlane_d(s, 0) + readlane_d(s, 16), b = readlane_d(s, 32) + readlane_d(s, 48);
+            s = sub ? b : a;
+        }
+        if (isq[i] ? gq != nullptr : gk != nullptr) {
+            const float4 gv = isq[i] ? g0 : g1;
+            const float inv = (float)rsqrt_f64(div_rcp(s, (double)HD, 1.0 / HD) + (double)eps);
+            x = make_float4(x.x * inv * gv.x, x.y * inv * gv.y, x.z * inv * gv.z, x.w * inv * gv.w);
+        }
+        const float e[4] = {x.x, x.y, x.z, x.w};
+        float o[4];
+        if (neox) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const float cc = co[2 * q], si = sn[2 * q];
+                o[2 * q] = e[2 * q] * cc - e[2 * q + 1] * si;
+                o[2 * q + 1] = e[2 * q] * si + e[2 * q + 1] * cc;
+            }
+        } else {
+            float pe[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) pe[q] = __shfl(e[q], lo ? lane + NL / 2 : lane - NL / 2);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const float cc = co[q], si = sn[q];
+                o[q] = lo ? e[q] * cc - pe[q] * si : pe[q] * si + e[q] * cc;
+            }
+        }
+        v[i] = make_float4(o[0], o[1], o[2], o[3]);
+    }
+#pragma unroll
+    for (int i = 0; i < kTokRows; i++)
+        if (out[i]) *reinterpret_cast<float4*>(out[i]) = v[i];
+}
+
 int launch_norm_rope_rows(hipStream_t s, const float* x, float* y, int rows, int heads, int hd, const float* g,
                           float eps, int start_pos, const float* cosT, const float* sinT, int neox) {
     if (rows == 0) return GORCH_HIP_OK;
@@ -176,6 +262,20 @@ int launch_norm_rope_rows2(hipStream_t s, const float* xq, float* yq, int rows_q
                            int start_pos, const float* cosT, const float* sinT, int neox, const int* pos_dev,
                            long long yk_pos_stride) {
     if (rows_q + rows_k == 0) return GORCH_HIP_OK;
+    // a prompt (host position): one block per token; fewer tokens leave CUs
+    // idle that the row form uses
+    const int toks = rows_q / heads_q;
+    if (!pos_dev && (hd == 64 || hd == 128) && toks >= 64 && toks == rows_k / heads_k &&
+        heads_q + heads_k <= 4 * kTokRows * (256 / hd)) {
+        if (hd == 64)
+            hipLaunchKernelGGL(k_norm_rope_tok<16>, dim3(toks), dim3(256), 0, s, xq, yq, heads_q, gq, xk, yk, heads_k, gk,
+                               eps, start_pos, cosT, sinT, neox);
+        else
+            hipLaunchKernelGGL(k_norm_rope_tok<32>, dim3(toks), dim3(256), 0, s, xq, yq, heads_q, gq, xk, yk, heads_k, gk,
+                               eps, start_pos, cosT, sinT, neox);
+        count(CNT_ELEMENTWISE);
+        return check_launch("norm_rope_tok");
+    }
     hipLaunchKernelGGL(k_norm_rope_rows, dim3((rows_q + rows_k + 3) / 4), dim3(256), 0, s, xq, yq, rows_q, heads_q,
                        hd, gq, eps, start_pos, cosT, sinT, neox, xk, yk, rows_k, heads_k, gk, pos_dev, yk_pos_stride);
     count(CNT_ELEMENTWISE);
