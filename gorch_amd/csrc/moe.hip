@@ -89,12 +89,8 @@ static size_t moe_layout(int M, int dim, int ffn, int E, int K, char* base, MoeW
 // never selected; a load under a branch would be waited on before the
 // next one, one round trip per expert). M * E < 2^29 (host check).
 template <int EV, int KT>
-__device__ __forceinline__ void moe_topk_token(__amdgpu_buffer_rsrc_t rl, int tok, int E, int K, int (&idx)[KT],
-                                               float (&wgt)[KT]) {
-    float lv[EV];
-#pragma unroll
-    for (int j = 0; j < EV; j++)
-        lv[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rl, (tok * E + j) * 4, 0, 0));
+__device__ __forceinline__ void moe_topk_values(const float (&lv)[EV], int E, int K, int (&idx)[KT],
+                                                float (&wgt)[KT]) {
     float val[KT];
     unsigned long long taken = 0ull;
 #pragma unroll
@@ -132,6 +128,15 @@ __device__ __forceinline__ void moe_topk_token(__amdgpu_buffer_rsrc_t rl, int to
     }
 #pragma unroll
     for (int s = 0; s < KT; s++) wgt[s] = s < K ? e_[s] / sum : 0.f;
+}
+template <int EV, int KT>
+__device__ __forceinline__ void moe_topk_token(__amdgpu_buffer_rsrc_t rl, int tok, int E, int K, int (&idx)[KT],
+                                               float (&wgt)[KT]) {
+    float lv[EV];
+#pragma unroll
+    for (int j = 0; j < EV; j++)
+        lv[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rl, (tok * E + j) * 4, 0, 0));
+    moe_topk_values<EV, KT>(lv, E, K, idx, wgt);
 }
 
 template <int EV>
@@ -302,6 +307,117 @@ __global__ __launch_bounds__(kRouteThreads) void k_moe_route(int M, int E, int K
             ws.perm_w[p] = ws.topw[a];
             ws.inv[a] = p;
         }
+}
+
+// The router Linear, top-K and grouping of a decode batch (up to 64 tokens, 8
+// experts, top-2) in one block: 16 waves split the columns of x and of the
+// router in 32-wide matrix-core steps (x as three bf16 terms, f32-level
+// products), their partial logits are added in LDS in wave order, then lane t
+// of the first wave takes token t's top-K and the expert groups come from
+// that wave's ballots, stable in token order as k_moe_route's. Replaces a
+// K-split GEMV, its epilogue and k_moe_route: three launches and their
+// latency, 11 us for 16 KB of router. (A wave per token, reading the router
+// rows again for each, gained nothing at 16 tokens.)
+constexpr int kFrontTokens = 64, kFrontE = 8;
+__global__ __launch_bounds__(1024) void k_moe_front(const float* __restrict__ x, const uint16_t* __restrict__ wr,
+                                                    const float* __restrict__ br, int M, int d, int E, int K, MoeWs ws,
+                                                    int* topi_out, float* topw_out) {
+    constexpr int MT = kFrontTokens / 16;
+    __shared__ float part[16][kFrontTokens][kFrontE];
+    __shared__ float lg[kFrontTokens][kFrontE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4, mt = (M + 15) / 16;
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(x, (long long)M * d * 4), rw = make_rsrc(wr, (long long)E * d * 2);
+    floatx4 acc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int s = wave; s * 32 < d; s += 16) {
+        // rows past M or E and columns past d read zeros (past the resource
+        // or an out-of-range offset)
+        const int k = 32 * s + 8 * g;
+        const bf16x8 w = __builtin_bit_cast(
+            bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rw, k < d && r < E ? (r * d + k) * 2 : kOutOfRange, 0, 0));
+        float4 u[MT], v[MT];
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            const int row = 16 * i + r, off = i < mt && k < d && row < M ? (row * d + k) * 4 : kOutOfRange;
+            u[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
+            v[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rx, off + 16, 0, 0));
+        }
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            const float f[8] = {u[i].x, u[i].y, u[i].z, u[i].w, v[i].x, v[i].y, v[i].z, v[i].w};
+            bf16x8 hi, mid, lo;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const uint32_t h = __float_as_uint(f[e]) & 0xffff0000u;
+                const float r1 = f[e] - __uint_as_float(h);
+                const uint32_t m = __float_as_uint(r1) & 0xffff0000u;
+                hi[e] = __builtin_bit_cast(__bf16, (uint16_t)(h >> 16));
+                mid[e] = __builtin_bit_cast(__bf16, (uint16_t)(m >> 16));
+                lo[e] = (__bf16)(r1 - __uint_as_float(m));
+            }
+            acc[i] = mfma16x16x32(hi, w, acc[i]);
+            acc[i] = mfma16x16x32(mid, w, acc[i]);
+            acc[i] = mfma16x16x32(lo, w, acc[i]);
+        }
+    }
+    // lane (r, g): tokens 4g .. 4g + 3, expert r of each 16-token tile
+    if (r < kFrontE)
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) part[wave][16 * i + 4 * g + q][r] = acc[i][q];
+    __syncthreads();
+    if (threadIdx.x < kFrontTokens * kFrontE) {
+        const int t = threadIdx.x / kFrontE, e = threadIdx.x % kFrontE;
+        float s = part[0][t][e];
+#pragma unroll
+        for (int q = 1; q < 16; q++) s += part[q][t][e];
+        lg[t][e] = br && e < E ? s + br[e] : s;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    const bool live = lane < M;
+    float lv[kFrontE];
+#pragma unroll
+    for (int e = 0; e < kFrontE; e++) lv[e] = live && e < E ? lg[lane][e] : 0.f;
+    int idx[2];
+    float wv[2];
+    moe_topk_values<kFrontE, 2>(lv, E, K, idx, wv);
+    if (!live || K < 2) idx[1] = -1;
+    if (!live) idx[0] = -1;
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    int base = 0, nt = 0, pos[2] = {0, 0};
+#pragma unroll
+    for (int e = 0; e < kFrontE; e++) {
+        if (e >= E) break;
+        const unsigned long long bits = __ballot(idx[0] == e || idx[1] == e);
+        const int n = __popcll(bits), p = base + __popcll(bits & lt);
+        if (idx[0] == e) pos[0] = p;
+        if (idx[1] == e) pos[1] = p;
+        if (n && lane == 0) {  // one tile: n <= 64 rows
+            ws.tile_e[nt] = e;
+            ws.tile_r0[nt] = base;
+            ws.tile_n[nt] = n;
+        }
+        nt += n != 0;
+        base += n;
+    }
+    if (lane == 0) *ws.ntiles = nt;
+    if (!live) return;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        if (s >= K) break;
+        const size_t a = (size_t)lane * K + s;
+        ws.topi[a] = idx[s];
+        ws.topw[a] = wv[s];
+        if (topi_out) topi_out[a] = idx[s];
+        if (topw_out) topw_out[a] = wv[s];
+        ws.perm_tok[pos[s]] = lane;
+        ws.perm_w[pos[s]] = wv[s];
+        ws.inv[a] = pos[s];
+    }
 }
 
 // out[t] = sum over the token's K packed rows in ascending expert order
@@ -806,7 +922,13 @@ extern "C" int gorch_hip_moe_forward(void* stream, const gorch_hip_moe_weights* 
     moe_layout(M, d, F, E, K, (char*)workspace, &ws);
     hipStream_t s = stream_of(stream);
     const float* lg = logits;
-    if (!lg) {
+    // a decode batch: router, top-K and grouping in one launch
+    const bool front = !lg && M <= kFrontTokens && E <= kFrontE && K <= 2 && (uintptr_t)x % 16 == 0 &&
+                       (uintptr_t)w->wr % 16 == 0;
+    if (front) {
+        hipLaunchKernelGGL(k_moe_front, dim3(1), dim3(1024), 0, s, x, w->wr, w->br, M, d, E, K, ws, topk_idx, topk_w);
+        GH_TRY(check_launch("moe_front"));
+    } else if (!lg) {
         GH_TRY(launch_linear_bf16(s, x, w->wr, w->br, nullptr, ws.logits, M, E, d, GORCH_HIP_EPI_NONE));
         lg = ws.logits;
     }
@@ -814,7 +936,8 @@ extern "C" int gorch_hip_moe_forward(void* stream, const gorch_hip_moe_weights* 
     // top-K slots sized to K (every absent slot still costs its compares).
     // Up to two slots, 8 experts and 4096 tokens: the routing block takes
     // the top-K itself (one launch fewer)
-    if (K <= 2 && E <= 8 && M <= 4 * kRouteThreads) {
+    if (front) {
+    } else if (K <= 2 && E <= 8 && M <= 4 * kRouteThreads) {
         hipLaunchKernelGGL((k_moe_route<2, 8>), dim3(1), dim3(kRouteThreads), 0, s, M, E, K, tile_rows, ws, lg,
                            topk_idx, topk_w);
     } else {

@@ -51,3 +51,28 @@ def test_moe_few_rows(gpu, M, dim, ffn, E, K, skew):
     out, _, _ = gpu.MoE(w).forward(dev(x), dev(logits))
     ref = reference(w, x, logits)
     assert np.linalg.norm(out.cpu().numpy() - ref) <= 2e-5 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("M,dim,E,K", [(1, 40, 1, 1), (15, 1032, 5, 2), (16, 64, 8, 2), (17, 520, 8, 1), (64, 264, 7, 2),
+                                       (65, 264, 7, 2), (33, 2056, 2, 2)])
+def test_moe_router_batch(gpu, M, dim, E, K):
+    """The router, top-K and grouping of a decode batch in one launch (up to
+    64 tokens; 65 takes the Linear and the routing block): choices and weights
+    from float64 logits (the seeds keep every top-K gap above 1e-4), 5e-5 on
+    the weights (at 65 tokens two bf16 terms, 2^-16 of a |x||w| sum of 4, a
+    quarter of it through the softmax: 1.6e-5; three terms below)."""
+    x, _, w = syn.moe_inputs(M=M, dim=dim, ffn=64, experts=E, top_k=K, seed=3 * M + E, with_router=True)
+    rng = np.random.default_rng(M)
+    w["br"] = rng.standard_normal(E).astype(np.float32)
+    logits = x.astype(np.float64) @ bf16_to_f32(w["wr"]).astype(np.float64).T + w["br"]
+    if K < E:
+        s = -np.sort(-logits, axis=1)
+        assert (s[:, K - 1] - s[:, K]).min() > 1e-4
+    out, idx, wts = gpu.MoE(w).forward(torch.from_numpy(x).cuda())
+    order = np.argsort(-logits, axis=1, kind="stable")[:, :K]
+    val = np.take_along_axis(logits, order, 1)
+    p = np.exp(val - val.max(1, keepdims=True))
+    assert np.array_equal(idx.cpu().numpy(), order)
+    assert np.abs(wts.cpu().numpy() - p / p.sum(1, keepdims=True)).max() <= 5e-5
+    ref = reference(w, x, logits)
+    assert np.linalg.norm(out.cpu().numpy() - ref) <= 3e-5 * np.linalg.norm(ref)
