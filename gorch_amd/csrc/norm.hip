@@ -46,6 +46,64 @@ __global__ __launch_bounds__(256) void k_layernorm(const float* __restrict__ x, 
     }
 }
 
+// Rows of at most 1024 R floats (N % 4 == 0, 16-byte rows and gains): a block
+// per row holds it in registers, R float4 a thread, so the two f64 passes
+// (mean, then squared deviations) and the output cost one trip to memory
+// instead of three; the gains are requested with the row. Same statistics
+// and f32 operations as k_layernorm. Latency for few rows (64 x 768: 3.5 ->
+// 2.5 us in a graph), HBM for many (8192 x 1600: 33.8 -> 16.8 us, 6.3 TB/s).
+template <int R>
+__global__ __launch_bounds__(256) void k_layernorm_rows(const float* __restrict__ x, const float* __restrict__ g,
+                                                        const float* __restrict__ b, float* __restrict__ y, int N,
+                                                        float eps, long long in_stride) {
+    __shared__ double sh[8];
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(x + (size_t)blockIdx.x * in_stride, (long long)N * 4);
+    const __amdgpu_buffer_rsrc_t rg = make_rsrc(g, (long long)N * 4), rb = make_rsrc(b, (long long)N * 4);
+    auto ld = [](__amdgpu_buffer_rsrc_t r, int off) {
+        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    };
+    float4 v[R], gv[R], bv[R];
+#pragma unroll
+    for (int c = 0; c < R; c++) {
+        const int off = 16 * ((int)threadIdx.x + 256 * c);  // past N: zeros
+        v[c] = ld(rx, off);
+        gv[c] = ld(rg, off);
+        bv[c] = ld(rb, off);
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // sum over the block: 4 waves, in wave order
+    auto total = [&](double s, double* buf) {
+        s = wave_sum_d(s);
+        if (lane == 0) buf[wave] = s;
+        __syncthreads();
+        return ((buf[0] + buf[1]) + buf[2]) + buf[3];
+    };
+    const double rn = 1.0 / N;
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < R; c++) s += ((double)v[c].x + (double)v[c].y) + ((double)v[c].z + (double)v[c].w);
+    const double mean = div_rcp(total(s, sh), (double)N, rn);
+    double q = 0.0;
+#pragma unroll
+    for (int c = 0; c < R; c++) {
+        if (4 * ((int)threadIdx.x + 256 * c) >= N) continue;
+        const double d0 = (double)v[c].x - mean, d1 = (double)v[c].y - mean, d2 = (double)v[c].z - mean,
+                     d3 = (double)v[c].w - mean;
+        q += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
+    }
+    const double var = div_rcp(total(q, sh + 4), (double)N, rn);
+    const float inv = (float)rsqrt_f64(var + (double)eps), fm = (float)mean;
+    float* out = y + (size_t)blockIdx.x * N;
+#pragma unroll
+    for (int c = 0; c < R; c++) {
+        const int j = 4 * ((int)threadIdx.x + 256 * c);
+        if (j >= N) continue;
+        const float n0 = (v[c].x - fm) * inv, n1 = (v[c].y - fm) * inv, n2 = (v[c].z - fm) * inv, n3 = (v[c].w - fm) * inv;
+        *reinterpret_cast<float4*>(out + j) =
+            make_float4(n0 * gv[c].x + bv[c].x, n1 * gv[c].y + bv[c].y, n2 * gv[c].z + bv[c].z, n3 * gv[c].w + bv[c].w);
+    }
+}
+
 // (also used in place by the GQA qk-norm: each thread rewrites only the
 // elements it read after the row's sum is complete)
 __global__ __launch_bounds__(256) void k_rmsnorm(const float* x, const float* __restrict__ g, float* y, int N,
@@ -289,6 +347,16 @@ int launch_reduce_rows(hipStream_t s, const float* part, int S, const float* bia
 int launch_layernorm(hipStream_t s, const float* x, const float* g, const float* b, float* y, int M, int N,
                      float eps, long long in_stride) {
     if (M == 0) return GORCH_HIP_OK;
+    const bool aligned = N % 4 == 0 && in_stride % 4 == 0 &&
+                         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) % 16) == 0;
+    if (aligned && N <= 2048) {
+        if (N <= 1024)
+            hipLaunchKernelGGL(k_layernorm_rows<1>, dim3(M), dim3(256), 0, s, x, g, b, y, N, eps, in_stride);
+        else
+            hipLaunchKernelGGL(k_layernorm_rows<2>, dim3(M), dim3(256), 0, s, x, g, b, y, N, eps, in_stride);
+        count(CNT_NORM);
+        return check_launch("layernorm");
+    }
     hipLaunchKernelGGL(k_layernorm, dim3(M), dim3(256), 0, s, x, g, b, y, N, eps, in_stride);
     count(CNT_NORM);
     return check_launch("layernorm");
