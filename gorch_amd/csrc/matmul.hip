@@ -339,7 +339,8 @@ __global__ __launch_bounds__(256 * G, G <= 2 ? 2 : 1) void k_mm(const void* __re
     }
 }
 
-template <int T, int G>
+// HALF: two bf16 operands only (4 groups of 64 x 64 stages fit LDS then).
+template <int T, int G, bool HALF = false>
 static void launch_mm_t(hipStream_t s, const void* A, const void* B, float* C, int M, int N, int K, int batch,
                         bool ka, bool fa, bool kb, bool fb) {
     const unsigned gx = (N + T - 1) / T, gy = (M + T - 1) / T;
@@ -349,7 +350,8 @@ static void launch_mm_t(hipStream_t s, const void* A, const void* B, float* C, i
     hipLaunchKernelGGL((k_mm<T, G, T == 128 && (FA || FB) ? 32 : 64, KA, FA, KB, FB>), grid, dim3(256 * G), 0, s, A, B, C, M, N, K, xcd_map)
 #define GH_MM_T(KA, KB)                              \
     do {                                             \
-        if (fa && fb) GH_MM(KA, true, KB, true);     \
+        if constexpr (HALF) GH_MM(KA, false, KB, false); \
+        else if (fa && fb) GH_MM(KA, true, KB, true); \
         else if (fa) GH_MM(KA, true, KB, false);     \
         else if (fb) GH_MM(KA, false, KB, true);     \
         else GH_MM(KA, false, KB, false);            \
@@ -367,8 +369,9 @@ static void launch_mm_t(hipStream_t s, const void* A, const void* B, float* C, i
 //     K steps on each: 64 x 64 x 2048 ff 15.1 against 37.6 (64/2), 47.9
 //     (64/1); 1103 x 65 x 1699 ff 14.9 / 33.0 / 42.3; 512^3 hh 3.6 / 4.9 /
 //     5.2; but 128 tiles (8 x 200^2 x 200 fh) 7.2 / 5.9 / 6.6.
-//   n64 <= 256: 64 x 64, 2 groups, one block per CU: 1024^3 hh 9.5 against
-//     11.9 (64/1) and 14.0 (32/4), ff 23.0 / 26.6 / 34.6.
+//   n64 <= 256: 64 x 64, 2 groups, one block per CU: 1024^3 ff 23.0 against
+//     26.6 (64/1) and 34.6 (32/4); two bf16 operands leave LDS for 4 groups,
+//     which pay from a few steps each: hh 8.7 / 9.5 (64/2) / 11.9 / 14.0.
 //   else 64 x 64, 1 group: 2048^3 hh 39.6 against 41.4 (64/2), 45.2 (128/1);
 //     30 x 92 x 725 x 687 ff 41.7 / 50.3 / 50.9.
 //   128 x 128 from 512 such tiles: half the operand traffic, 4096^3 hh 165
@@ -380,6 +383,7 @@ static void launch_mm(hipStream_t s, const void* A, const void* B, float* C, int
     const long long n64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * batch;
     const long long n128 = (long long)((M + 127) / 128) * ((N + 127) / 128) * batch;
     if (n64 <= 64) launch_mm_t<32, 4>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
+    else if (n64 <= 256 && !fa && !fb && K >= 512) launch_mm_t<64, 4, true>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
     else if (n64 <= 256) launch_mm_t<64, 2>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
     else if (n128 < 512) launch_mm_t<64, 1>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
     else launch_mm_t<128, 1>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);

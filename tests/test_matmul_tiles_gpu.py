@@ -20,7 +20,7 @@ LAYOUTS = [(False, True), (False, False), (True, False)]
 DTYPES = [(True, True), (False, True), (False, False), (True, False)]
 SIZES = [
     (1, 1, 1, 1), (1, 1, 3, 9), (1, 2, 5, 64), (1, 33, 65, 127), (1, 64, 36, 256),   # 32 x 32 tiles, 4 groups
-    (3, 259, 290, 65), (1, 576, 512, 128), (70, 3, 2, 40),                           # 64 x 64, 2 groups
+    (3, 259, 290, 65), (1, 576, 512, 128), (70, 3, 2, 40), (1, 1000, 700, 577),      # 64 x 64, 2 groups (4: bf16)
     (1, 1090, 1028, 63), (5, 512, 449, 192),                                         # 64 x 64, 1 group
     (1, 2050, 4037, 33), (32, 515, 500, 64),                                         # 128 x 128
 ]
