@@ -511,8 +511,8 @@ __global__ void k_moe_combine(const float* __restrict__ yg, const int* __restric
 // lo to ~2^-16 relative, the split the MFMA kernels use) in the space of the
 // f32 Xg, and GEMM 1's epilogue writes H the same way, so both GEMMs load
 // 16-byte bf16 words only. Rows are grouped in 128-row tiles. The down GEMM
-// keeps 256-wide tiles although at d = 1024 that leaves half the CUs idle:
-// 128-wide tiles on every CU measured slower (148 vs 121 us, 2048 tokens).
+// takes 256-wide tiles where 128-wide ones would need a second round of CUs
+// (2048 tokens at d = 1024: 97 us on 144 blocks, 113 on 288).
 // Splitting the down GEMM's K over twice the blocks (raw partials, summed
 // with bias and routing weight by the combine) measured within noise of the
 // unsplit kernel (118 vs 121 us): these GEMMs are bound by the traffic from
@@ -1008,6 +1008,12 @@ extern "C" int gorch_hip_moe_forward(void* stream, const gorch_hip_moe_weights* 
             hipLaunchKernelGGL((k_moe_kw<false, 32, 64, 4, 2>), dim3((d + 63) / 64, max_tiles, chunks(32)), dim3(256), 0, s,
                                hhi, hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, ws);
         GH_TRY(check_launch("moe_kw_down"));
+    } else if (live * ((d + 127) / 128) <= 256) {
+        // 128-wide tiles while they still fit one round of CUs: 1024 tokens
+        // 201 -> 182 us a layer; past a round the 256-wide ones (2048 tokens,
+        // ~288 of these: 288 against 281)
+        GH_TRY((launch_moe_wide<false, 128>(s, dim3((d + 127) / 128, max_tiles, nsl), hhi, hlo, w->wdown, nullptr,
+                                            w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, cslice, ws)));
     } else {
         GH_TRY((launch_moe_wide<false, kWideBNDown>(s, dim3((d + kWideBNDown - 1) / kWideBNDown, max_tiles, nsl), hhi,
                                                     hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr,
