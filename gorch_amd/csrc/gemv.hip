@@ -1496,7 +1496,7 @@ static int launch_mfma_gemv(hipStream_t s, const float* x, const uint16_t* W, co
 }
 
 
-// M <= 16: the weight-streaming GEMV below; larger M: the tiled MFMA GEMM
+// M <= 16: the weight-streaming GEMV below; larger M: the tiled MFMA GEMMs
 // (gemm.hip), which re-reads each weight tile only once per BM rows.
 int launch_linear_bf16_od(hipStream_t s, const float* x, const uint16_t* W, const float* bias,
                           const float* residual, const OutDesc& od, int M, int N, int K, int epilogue,

@@ -17,6 +17,8 @@
 //   grouped GEMM 2   Yg = (H We_down^T + bd) * w(row), the routing weight
 //                    applied in the epilogue (the reference's Mul);
 //   k_moe_combine    out[t] = sum of the token's rows in ascending expert order.
+// Decode batches run router, top-K and routing in one launch (k_moe_front),
+// and few rows per expert take K-split tiles (k_moe_kw) in either grouped GEMM.
 // Expert weights are stacked [E][out][in] bf16 in one device array each.
 #include <algorithm>
 

@@ -3,9 +3,9 @@
 //
 // One 256-thread block per row. Statistics accumulate in f64 exactly as the
 // reference's CPU loops do (mean and variance for LayerNorm, sum of squares
-// for RMSNorm); the row stays in L1/L2 between the two passes. The inverse
-// is rounded to f32 and the output computed in f32 in the reference's
-// operand order.
+// for RMSNorm); the row stays in L1/L2 between the two passes
+// (k_layernorm_rows: in registers). The inverse is rounded to f32 and the
+// output computed in f32 in the reference's operand order.
 #include "common.h"
 
 namespace gh {
