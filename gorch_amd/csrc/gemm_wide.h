@@ -43,12 +43,17 @@ struct WideGemm {
     static constexpr int WM = BM / WGM, WNW = BNW / WGN;
     static constexpr int TM = WM / 16, TN = WNW / 16;
     static constexpr int A_U4 = NA * BM * CH / kThreads;  // 16-byte loads per thread per stage
-    static constexpr int W_U4 = NB * BNW * CH / kThreads;
+    // weight rows a stage holds: BNW, for one weight rounded up to whole load
+    // instructions (192 columns on 1024 threads: 256 rows, the last 64 zeros
+    // that cost no memory traffic and that no fragment reads)
+    static constexpr int RPL = kThreads / CH;
+    static constexpr int BNL = NB == 1 ? (BNW + RPL - 1) / RPL * RPL : BNW;
+    static constexpr int W_U4 = NB * BNL * CH / kThreads;
     static_assert(BK == 32 || BK == 64, "stage width");
     static_assert(A_U4 >= 1 && W_U4 >= 1 && TM >= 1 && TN >= 1, "tile too small");
-    static_assert(NA * BM * CH % kThreads == 0 && NB * BNW * CH % kThreads == 0, "uneven loads");
+    static_assert(NA * BM * CH % kThreads == 0 && NB * BNL * CH % kThreads == 0, "uneven loads");
     // each load instruction stays inside one plane / weight (uniform resource)
-    static_assert((BM * CH) % kThreads == 0 && (BNW * CH) % kThreads == 0, "plane split across a load");
+    static_assert((BM * CH) % kThreads == 0 && (BNL * CH) % kThreads == 0, "plane split across a load");
 
     // Chunk c of LDS row `row` sits at c ^ (row & 7) (64-wide rows) or
     // c ^ ((row >> 1) & 3) (32-wide rows): conflict-free for both the row
@@ -59,7 +64,7 @@ struct WideGemm {
 
     struct Smem {
         uint16_t a[2][NA][BM][BK];
-        uint16_t w[2][NB][BNW][BK];
+        uint16_t w[2][NB][BNL][BK];
     };
 
     // a[p] + row * lda: row of plane p (nrows valid); w[b] + n * K: column n
@@ -99,9 +104,9 @@ struct WideGemm {
 #pragma unroll
             for (int i = 0; i < W_U4; i++) {
                 const int idx = tid + kThreads * i;
-                const int b = kThreads * i / (BNW * CH), rem = idx % (BNW * CH), row = rem / CH, c = rem % CH;
+                const int b = kThreads * i / (BNL * CH), rem = idx % (BNL * CH), row = rem / CH, c = rem % CH;
                 const int k = k0 + 8 * c;
-                const int off = k < ke ? (min(row, ncols - 1) * K + k) * 2 : kOutOfRange;
+                const int off = k < ke && (BNL == BNW || row < BNW) ? (min(row, ncols - 1) * K + k) * 2 : kOutOfRange;
                 wr[i] = __builtin_amdgcn_raw_buffer_load_b128(rsw[b], off, 0, 0);
             }
         };
@@ -115,7 +120,7 @@ struct WideGemm {
 #pragma unroll
             for (int i = 0; i < W_U4; i++) {
                 const int idx = tid + kThreads * i;
-                const int b = kThreads * i / (BNW * CH), rem = idx % (BNW * CH), row = rem / CH, c = rem % CH;
+                const int b = kThreads * i / (BNL * CH), rem = idx % (BNL * CH), row = rem / CH, c = rem % CH;
                 *reinterpret_cast<u32x4*>(&sm.w[buf][b][row][8 * swz(row, c)]) = wr[i];
             }
         };

@@ -39,8 +39,8 @@ def reference(w, x, logits):
     (1, 64, 64, 4, 1, 0), (1, 72, 104, 8, 2, 0), (16, 264, 520, 8, 2, 0), (16, 64, 2056, 8, 2, 99), (33, 128, 192, 4, 2, 0),
     (70, 1032, 136, 8, 2, 0), (64, 512, 1368, 4, 2, 0), (150, 96, 264, 4, 2, 99), (300, 200, 328, 4, 2, 0),
     (129, 64, 4096, 2, 1, 0), (700, 320, 256, 8, 2, 1), (31, 40, 24, 64, 8, 0),
-    # more rows: the 128- and 256-wide down tiles
-    (1000, 1032, 136, 4, 2, 0), (1500, 1288, 72, 4, 2, 0), (2048, 1544, 64, 8, 2, 0),
+    # more rows: the 128-, 192- and 256-wide down tiles
+    (1000, 1032, 136, 4, 2, 0), (1500, 1288, 72, 4, 2, 0), (900, 1544, 136, 8, 2, 0), (2048, 1544, 64, 8, 2, 0),
 ])
 def test_moe_few_rows(gpu, M, dim, ffn, E, K, skew):
     """skew pushes tokens towards expert 0 (99: every token's first choice)."""
