@@ -88,7 +88,7 @@ __device__ __forceinline__ void gemm_epilogue(floatx4 (&acc)[TM][TN], const floa
             for (int v = 0; v < 4; v++) {
                 // bn is zero without a bias (a select here costs ~0.2 us)
                 float s = acc[i][j][v] + bn[j];
-                if constexpr (GELU) s = gelu_tanh(s);
+                if constexpr (GELU) s = gelu_gemm(s);
                 if constexpr (RES) s = res[i][j][v] + s;
                 acc[i][j][v] = s;
             }
@@ -342,7 +342,7 @@ struct Out4 {
         f4u o = {acc[0] + b[0], acc[1] + b[1], acc[2] + b[2], acc[3] + b[3]};
         if (epilogue == GORCH_HIP_EPI_GELU)
 #pragma unroll
-            for (int v = 0; v < 4; v++) o[v] = gelu_fast(o[v]);
+            for (int v = 0; v < 4; v++) o[v] = gelu_gemm(o[v]);
         return r + o;
     }
     __device__ __forceinline__ void put(int m, int n, const f4u& s) const {
