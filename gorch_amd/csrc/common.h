@@ -402,6 +402,8 @@ bool gemv_pair_swiglu_ok(int F, int K);
 // The gate/up product of more than 16 rows with SwiGLU in its epilogue
 // (gemm.hip): y [M, N] from x [M, K] and W [2N, K].
 bool gemm_pair_swiglu_ok(int M, int N, int K);
+// Names for gorch_hip_kernel_choice.
+const char* gemm_choice_name(int M, int N, int K, bool act_bf16);
 int launch_gemm_pair_swiglu(hipStream_t s, const float* x, const uint16_t* W, float* y, int M, int N, int K);
 int launch_swiglu(hipStream_t s, const float* g, const float* v, float* y, int64_t n);
 
@@ -563,8 +565,8 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 // 3.8 (3.7), 3.9 (3.8), 3.7 (4.1), 2.8 (3.8), 2.1 (2.8); for negative x alone
 // 7.8 (36: 1 + tanh cancels there). x / (1 + exp(-2u)) on the same two
 // instructions has 4.7 (3.8) at 1. Linears with GELU against tanhf: 512 x 768 x
-// 3072 14.1 -> 13.0 us (64-row tiles); against that shorter form 8192 x 1600 x
-// 6400 306 -> 312 (256-row tiles). The GEMVs keep tanhf: it is not on their
+// 3072 14.1 -> 13.0 us (64-row tiles); against that shorter form 8192 x 768 x
+// 3072 81.5 -> 85.1, 8192 x 1600 x 6400 305 -> 306 (256-row tiles). The GEMVs keep tanhf: it is not on their
 // path's bound, and the tile GEMV compiled with a form like this ran slower
 // (LM head of 16 rows 15.8 -> 16.8 us).
 __device__ __forceinline__ float gelu_gemm(float x) {

@@ -3,7 +3,7 @@
 // with A f32 [M,K], W bf16 [N,K] (the nn.Linear layout, nn/module.go:61-88).
 //
 // Three kernels on v_mfma_f32_16x16x32_bf16, chosen by estimated time
-// (gemm_kind):
+// (gemm_choice):
 //   k_gemm_kw: few tiles (short prompts, narrow weights): the waves of a block
 //     split K, each through LDS stages of its own;
 //   k_gemm_db: 64-row tiles of 64, 96 or 128 columns on 2 x (2..4) waves of
@@ -522,10 +522,12 @@ __global__ __launch_bounds__(64 * G) void k_gemm_kw(const float* __restrict__ A,
 // together 236).
 // A wave waits for its own loads (vmcnt, all but the newest stage) before the
 // barrier behind which the next stage is first read.
-template <int TN, bool SPLIT, bool KT>
+// GELU is compiled in or out: decided at run time, its 64 TN / 4 copies in the
+// epilogue cost products without it up to 4% (8192 x 1024 x 6144 192 us, 185 so).
+template <int TN, bool SPLIT, bool KT, bool GELU>
 __global__ __launch_bounds__(512, 2) void k_gemm_pp(const float* __restrict__ A, const uint16_t* __restrict__ W,
                                                     const float* __restrict__ bias, const float* residual, OutDesc od,
-                                                    int M, int N, int K, int epilogue, int seg4, int band) {
+                                                    int M, int N, int K, int seg4, int band) {
     constexpr int TM = 4, BM = 256, BN = 32 * TN, NW = 8;
     constexpr int LA = BM / 8 / NW, LW = (BN / 16 + NW - 1) / NW;  // loads per wave and stage
     constexpr int kA = BM * 128, kStage = kA + LW * NW * 1024;     // bytes (W groups past BN: zeros, unread)
@@ -644,7 +646,8 @@ __global__ __launch_bounds__(512, 2) void k_gemm_pp(const float* __restrict__ A,
             for (int j = 0; j < TN; j++) rv[(i + 1) & 1][j] = out.res(mw + 16 * (i + 1), nw + 16 * j);
 #pragma unroll
         for (int j = 0; j < TN; j++)
-            out.put(mw + 16 * i, nw + 16 * j, out.value(acc[i][j], bv[j], rv[i & 1][j], epilogue));
+            out.put(mw + 16 * i, nw + 16 * j,
+                    out.value(acc[i][j], bv[j], rv[i & 1][j], GELU ? GORCH_HIP_EPI_GELU : GORCH_HIP_EPI_NONE));
     }
 }
 
@@ -662,16 +665,21 @@ static void launch_pp(hipStream_t s, const float* A, const uint16_t* W, const fl
     const int seg4 = segments_by_4(od);
     // bands of 4 tile rows per XCD: 8192 x 1600 x 6400 347 -> 328 us (8: 333)
     constexpr int band = 4;
-#define GH_PP(SP, KTV)                                                                                         \
-    hipLaunchKernelGGL((k_gemm_pp<TN, SP, KTV>), grid, dim3(512), 0, s, A, W, bias, residual, od, M, N, K, epilogue, \
-                       seg4, band)
+#define GH_PP(SP, KTV, GE)                                                                                      \
+    hipLaunchKernelGGL((k_gemm_pp<TN, SP, KTV, GE>), grid, dim3(512), 0, s, A, W, bias, residual, od, M, N, K, seg4, band)
+#define GH_PP_E(SP, KTV)                                          \
+    do {                                                          \
+        if (epilogue == GORCH_HIP_EPI_GELU) GH_PP(SP, KTV, true); \
+        else GH_PP(SP, KTV, false);                               \
+    } while (0)
     if (K % kStK) {
-        if (act_bf16) GH_PP(false, true);
-        else GH_PP(true, true);
+        if (act_bf16) GH_PP_E(false, true);
+        else GH_PP_E(true, true);
     } else {
-        if (act_bf16) GH_PP(false, false);
-        else GH_PP(true, false);
+        if (act_bf16) GH_PP_E(false, false);
+        else GH_PP_E(true, false);
     }
+#undef GH_PP_E
 #undef GH_PP
 }
 
@@ -693,11 +701,7 @@ static void launch_kw(hipStream_t s, const float* A, const uint16_t* W, const fl
 #undef GH_KW
 }
 
-// Tile width for k_gemm_db: the most 64-row blocks that still fit one
-// round on the chip (measured at 512 x 768: N = 2304 on 64 x 96, 192
-// blocks, 7.1 us; N = 3072 on 64 x 96, 256 blocks, 7.4 us, against 7.5 /
-// 7.6 us on 64 x 128), the widest when every width exceeds it.
-static int db_waves(int M, int N) {
+static int cu_count() {
     static const int cus = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -705,12 +709,20 @@ static int db_waves(int M, int N) {
             n = 256;
         return n;
     }();
+    return cus;
+}
+
+// Tile width for k_gemm_db: the most 64-row blocks that still fit one
+// round on the chip (measured at 512 x 768: N = 2304 on 64 x 96, 192
+// blocks, 7.1 us; N = 3072 on 64 x 96, 256 blocks, 7.4 us, against 7.5 /
+// 7.6 us on 64 x 128), the widest when every width exceeds it.
+static int db_waves(int M, int N) {
     const long long mb = (M + 63) / 64;
     int best = 4;
     long long best_blocks = 0;
     for (int w = 4; w >= 2; w--) {
         const long long blocks = mb * ((N + 32 * w - 1) / (32 * w));
-        if (blocks <= cus && blocks > best_blocks) {
+        if (blocks <= cu_count() && blocks > best_blocks) {
             best = w;
             best_blocks = blocks;
         }
@@ -749,53 +761,125 @@ static void launch_db(hipStream_t s, const float* A, const uint16_t* W, const fl
     }
 }
 
-// Kernel and tile by estimated time (us), each estimate fitted to measured
-// launches on 256 CUs with the weight beyond L2:
-//   k_gemm_db (64 rows x 32 w columns): 2.5 + steps of 64 x {0.56, 0.78, 0.83}
-//     (w = 2, 3, 4) x blocks / 256. 777 x 1024 x 4096 22.8 (estimate 24),
-//     777 x 1024 x 6144 32.4 (35), 8192 x 1600 x 1600 128 (138).
-//   k_gemm_kw (BM x BN, one block per CU): 1.5 + rounds x (3.5 + K (4 BM +
-//     2 BN) bytes at 75 B/ns), and at least 3.5 + all blocks' bytes at 13.5
-//     TB/s. 97 x 3072 x 768 7.8 on 16 x 32 tiles against 26.8 (db); 32 x 3072
-//     x 768 8.1 / 26.4; 777 x 3072 x 1024 22.5 on 64 x 64 / 29.1.
-//   k_gemm_pp (256 x 32 TN): 3 + rounds x max(steps of 32 x c(TN), the stores
-//     of one tile per CU, 1.86 TN). 8192 x 1600 x 6400 328 at TN = 7 (4 rounds; 348 at 8, 344 at 5)
-//     against 429 for the 128 x 128 tiles without a pipeline it replaced;
-//     2007 x 1600 x 4800 72 / 107 (db 95); 200 x 1600 x 50257 84 / 128.
+// Kernel and tile by estimated time. Each estimate (us) is a sum of terms
+// fitted (least squares on the relative error, near the fastest kernel) to
+// 1,474 measured launches of every kernel: 17 to 9,000 rows, K 32 to 12,288, N
+// 48 to 50,257, both activation modes, weights rotated so that large ones come
+// from HBM. n = blocks on the busiest CU, load = blocks per CU, k = K steps:
+//   k_gemm_db  a + b k ceil(n / blocks that fit a CU) + c k n + d k load
+//   k_gemm_kw  a + b n + c (steps of a wave) n
+//   k_gemm_pp  a + b n + c k n + d k load
+// each plus e per MB of operands that the XCDs read into their L2s (A once
+// per column tile and W once per row tile, 8 at most; k_gemm_pp's bands share
+// them) and f per MB written (f2 for k_gemm_db when N is no multiple of 4:
+// its rows then start off a 16-byte boundary).
+// The choice is on average 1.0% slower than the fastest kernel of a size. It is
+// more than 5% slower than k_gemm_db at 16 of 1,126 sizes of less than a round
+// of 128 x 128 tiles, 14% at most: the K-split tiles have to be 3% faster by
+// estimate. With fewer terms, one set for both activation modes
+// and no traffic term the average was 3.4%, and K-split tiles ran where
+// k_gemm_db is 1.2 to 1.6 times as fast: 777 x 1600 x 6400 80.6 us against
+// 61.5, 1400 x 896 x 4864 62.6 / 48.9, with bf16 activations 79.2 / 50.9 and
+// 60.4 / 38.8.
 enum GemmKind { kDb, kKw16x32, kKw32x32, kKw32x64, kKw64x64, kPp4, kPp5, kPp6, kPp7, kPp8 };
-static GemmKind gemm_kind(int M, int N, int K) {
+struct GemmChoice {
+    GemmKind kind;
+    double us;
+};
+static GemmChoice gemm_choice(int M, int N, int K, bool act_bf16) {
     auto cdiv = [](long long a, long long b) { return (a + b - 1) / b; };
-    constexpr double kCus = 256.0;
-    const int w = db_waves(M, N);
-    const double cdb[3] = {0.56, 0.78, 0.83};
-    GemmKind best = kDb;
-    double t = 2.5 + cdiv(K, 64) * cdb[w - 2] * std::max(1.0, cdiv(M, 64) * cdiv(N, 32 * w) / kCus);
-    auto take = [&](GemmKind k, double c) {
-        if (c < t) {
-            t = c;
-            best = k;
-        }
+    const double cus = cu_count(), mb = 1e-6;
+    const double out = 4 * mb * M * N;
+    auto traffic = [&](int bm, int bn) {
+        return mb * ((double)std::min(8ll, cdiv(N, bn)) * 4 * M * K + (double)std::min(8ll, cdiv(M, bm)) * 2 * N * K);
     };
-    const int kw[4][2] = {{16, 32}, {32, 32}, {32, 64}, {64, 64}};
-    for (int i = 0; i < 4; i++) {
-        const double blocks = (double)cdiv(M, kw[i][0]) * cdiv(N, kw[i][1]);
-        const double bytes = (double)K * (4 * kw[i][0] + 2 * kw[i][1]);
-        take((GemmKind)(kKw16x32 + i),
-             std::max(1.5 + std::ceil(blocks / kCus) * (3.5 + bytes / 75e3), 3.5 + blocks * bytes / 13.5e6));
+    // the grid's second dimension
+    auto rows_ok = [&](int bm) { return cdiv(M, bm) <= 65535; };
+    GemmChoice best{kDb, 1e30};
+    {
+        // a, b, c, d, e, f, f2 for 64, 96 and 128 columns; split, bf16 activations
+        constexpr double C[2][3][7] = {{{3.86, 0.241, 0.162, 0, 0.0427, 0.223, 0.287},
+                                        {3.88, 0, 0.535, 0.0288, 0.0192, 0.210, 0.250},
+                                        {4.01, 0.150, 0.360, 0.0336, 0.0223, 0.179, 0.270}},
+                                       {{3.67, 0.123, 0.163, 0, 0.0393, 0.164, 0.212},
+                                        {3.71, 0.0467, 0.268, 0, 0.0380, 0.196, 0.268},
+                                        {3.85, 0.0941, 0.224, 0, 0.0435, 0.167, 0.237}}};
+        constexpr int kFit[2][3] = {{2, 2, 2}, {4, 3, 2}};  // blocks that fit a CU (LDS)
+        const int w = db_waves(M, N);
+        const double* c = C[act_bf16][w - 2];
+        const double blocks = (double)cdiv(M, 64) * cdiv(N, 32 * w), n = std::ceil(blocks / cus), k = (double)cdiv(K, 64);
+        if (rows_ok(64))
+            best.us = c[0] + k * (c[1] * std::ceil(n / kFit[act_bf16][w - 2]) + c[2] * n + c[3] * blocks / cus) +
+                      c[4] * traffic(64, 32 * w) + out * (N % 4 == 0 ? c[5] : c[6]);
     }
-    const double cpp[5] = {1.05, 1.3, 1.43, 1.62, 1.8};
-    for (int tn = 4; tn <= 8; tn++) {
-        const double rounds = std::ceil((double)cdiv(M, 256) * cdiv(N, 32 * tn) / kCus);
-        take((GemmKind)(kPp4 + tn - 4), 3.0 + rounds * std::max(cdiv(K, 32) * cpp[tn - 4], 1.86 * tn));
+    // (`rank` orders the kernels: the estimate, raised for the K-split tiles)
+    double rank = best.us;
+    auto take = [&](GemmKind kind, double us, double r) {
+        if (r >= rank) return;
+        rank = r;
+        best = {kind, us};
+    };
+    {
+        constexpr int T[4][3] = {{16, 32, 8}, {32, 32, 8}, {32, 64, 4}, {64, 64, 4}};  // rows, columns, waves
+        constexpr double C[2][4][5] = {{{2.19, 1.18, 0.390, 0.0110, 0.715},              // a, b, c, e, f
+                                        {2.18, 1.74, 0.454, 0.0383, 0.373},
+                                        {2.47, 1.52, 0.395, 0.0294, 0.242},
+                                        {2.68, 2.47, 0.555, 0.0350, 0.208}},
+                                       {{2.17, 1.15, 0.393, 0.0061, 0.793},
+                                        {2.20, 1.67, 0.433, 0.0382, 0.406},
+                                        {2.42, 1.43, 0.390, 0.0277, 0.286},
+                                        {2.66, 2.33, 0.523, 0.0356, 0.125}}};
+        double kw = 1e30;
+        int at = 0;
+        for (int i = 0; i < 4; i++) {
+            const double n = std::ceil((double)cdiv(M, T[i][0]) * cdiv(N, T[i][1]) / cus);
+            const double* c = C[act_bf16][i];
+            const double us = c[0] + n * (c[1] + c[2] * cdiv(cdiv(K, kStK), T[i][2])) +
+                              c[3] * traffic(T[i][0], T[i][1]) + c[4] * out;
+            if (rows_ok(T[i][0]) && us < kw) {
+                kw = us;
+                at = i;
+            }
+        }
+        take((GemmKind)(kKw16x32 + at), kw, kw / 0.97);
+    }
+    // 256 rows of A, and of a residual, behind one 2 GiB resource
+    if (256ll * 4 * std::max(K, N) < kOutOfRange && rows_ok(256)) {
+        constexpr double C[2][5][5] = {{{3.86, 5.69, 0.520, 0.335, 0.0641},  // a, b, c, d, f for 4 to 8 column groups
+                                        {3.73, 5.73, 0.708, 0.309, 0.102},
+                                        {3.14, 7.75, 0.794, 0.329, 0.0979},
+                                        {2.36, 7.76, 0.971, 0.252, 0.154},
+                                        {0.584, 11.3, 1.01, 0.392, 0.139}},
+                                       {{4.20, 5.07, 0.520, 0.0783, 0.0775},
+                                        {3.83, 6.43, 0.543, 0.0942, 0.0855},
+                                        {3.16, 8.15, 0.563, 0.127, 0.0862},
+                                        {3.14, 7.53, 0.601, 0.139, 0.126},
+                                        {1.93, 10.0, 0.611, 0.185, 0.122}}};
+        for (int tn = 4; tn <= 8; tn++) {
+            const double* c = C[act_bf16][tn - 4];
+            const double blocks = (double)cdiv(M, 256) * cdiv(N, 32 * tn), n = std::ceil(blocks / cus);
+            const double k = (double)cdiv(K, kStK);
+            const double us = c[0] + n * (c[1] + c[2] * k) + c[3] * k * blocks / cus + c[4] * out;
+            take((GemmKind)(kPp4 + tn - 4), us, us);
+        }
     }
     return best;
+}
+
+// The kernel's name (gorch_hip_kernel_choice).
+const char* gemm_choice_name(int M, int N, int K, bool act_bf16) {
+    static const char* const kDbName[3] = {"db64x64", "db64x96", "db64x128"};
+    static const char* const kName[9] = {"kw16x32",   "kw32x32",   "kw32x64",   "kw64x64",  "pp256x128",
+                                         "pp256x160", "pp256x192", "pp256x224", "pp256x256"};
+    const GemmKind k = gemm_choice(M, N, K, act_bf16).kind;
+    return k == kDb ? kDbName[db_waves(M, N) - 2] : kName[k - kKw16x32];
 }
 
 // y[m, n] = silu(x W[n]) * (x W[N + n]) over a [2N, K] weight for more than 16
 // rows; false when the K-split tiles should take the product instead (few
 // tiles) or a weight panel spans 2 GiB.
 bool gemm_pair_swiglu_ok(int M, int N, int K) {
-    const GemmKind k = gemm_kind(M, 2 * N, K);
+    const GemmKind k = gemm_choice(M, 2 * N, K, false).kind;
     return M > 16 && !(k >= kKw16x32 && k <= kKw64x64) && (long long)2 * N * K * 2 < (1ll << 31);
 }
 int launch_gemm_pair_swiglu(hipStream_t s, const float* A, const uint16_t* W, float* y, int M, int N, int K) {
@@ -814,7 +898,7 @@ int launch_gemm_bf16w(hipStream_t s, const float* A, const uint16_t* W, const fl
                       const float* residual, const OutDesc& od, int M, int N, int K, int epilogue,
                       bool act_bf16) {
 #define GH_ARGS s, A, W, bias, residual, od, M, N, K, epilogue
-    switch (gemm_kind(M, N, K)) {
+    switch (gemm_choice(M, N, K, act_bf16).kind) {
         case kKw16x32: launch_kw<16, 32, 8, 3>(GH_ARGS, act_bf16); break;
         case kKw32x32: launch_kw<32, 32, 8, 3>(GH_ARGS, act_bf16); break;
         case kKw32x64: launch_kw<32, 64, 4, 3>(GH_ARGS, act_bf16); break;

@@ -480,6 +480,16 @@ int gorch_hip_read_dispatch_counts(uint64_t* out, int n) {
     return m;
 }
 
+const char* gorch_hip_kernel_choice(const char* op, const int* d, int n) {
+    if (!op || !d) return nullptr;
+    for (int i = 0; i < n; i++)
+        if (d[i] < 0) return nullptr;
+    const auto is = [&](const char* name, int count) { return n == count && !strcmp(op, name); };
+    if (is("linear", 4) && d[0] > 0 && d[1] > 0)
+        return gemm_choice_name(d[0], d[1], d[2], (d[3] & GORCH_HIP_LINEAR_ACT_BF16) != 0);
+    return nullptr;
+}
+
 void gorch_hip_reset_dispatch_counts(void) {
     for (int i = 0; i < CNT_COUNT; i++) g_counts[i].store(0, std::memory_order_relaxed);
 }

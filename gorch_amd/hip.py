@@ -69,6 +69,7 @@ SIGNATURES = {
     "gorch_hip_bf16_probe": (i32, []),
     "gorch_hip_read_dispatch_counts": (i32, [C.POINTER(C.c_uint64), i32]),
     "gorch_hip_reset_dispatch_counts": (None, []),
+    "gorch_hip_kernel_choice": (C.c_char_p, [C.c_char_p, C.POINTER(i32), i32]),
     "gorch_hip_bf16_to_f32": (i32, [vp, vp, vp, i64]),
     "gorch_hip_f32_to_bf16": (i32, [vp, vp, vp, i64]),
     "gorch_hip_matmul_dt": (i32, [vp, vp, vp, vp, u32, u32, u32, i32, i32, i32, i32]),
@@ -200,6 +201,12 @@ def dispatch_counts() -> dict:
 
 def reset_dispatch_counts() -> None:
     lib().gorch_hip_reset_dispatch_counts()
+
+
+def kernel_choice(op: str, *dims: int) -> str | None:
+    """The name of the kernel a call of these sizes launches (no device work)."""
+    name = lib().gorch_hip_kernel_choice(op.encode(), (i32 * len(dims))(*dims), len(dims))
+    return name.decode() if name else None
 
 
 def set_async(on: bool) -> None:

@@ -138,6 +138,13 @@ int gorch_hip_bf16_probe(void);
  * norm, elementwise, moe, argmax, codec; returns the number of slots. */
 int gorch_hip_read_dispatch_counts(uint64_t* out, int n);
 void gorch_hip_reset_dispatch_counts(void);
+/* The kernel that a call of these sizes launches, by name, for tests and
+ * profiles: no device work, static strings, NULL for an unknown op or sizes
+ * that launch nothing. op and dims:
+ *   "linear" {M, N, K, flags}: gorch_hip_linear_bf16_ex above 16 rows (any
+ *     number of rows with GORCH_HIP_LINEAR_ACT_BF16).
+ * The names are not an interface: they change with the kernels. */
+const char* gorch_hip_kernel_choice(const char* op, const int* dims, int n);
 
 /* ------------------------------------------------------------------------
  * bf16 codec on device (tensor.go:85-121; model/safetensors.go:164-184).

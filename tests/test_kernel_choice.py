@@ -1,0 +1,69 @@
+"""Which kernel a size runs (gorch_hip_kernel_choice), without a GPU: each rule
+of a dispatch at sizes where the kernels' measured times are far apart. The
+names listed with a size are the kernels within 15% of the fastest there
+(MI355X, HIP graphs, 256 CUs, which the library also assumes without a GPU).
+"""
+import pytest
+
+from gorch_amd import hip
+
+ACT = hip.LINEAR_ACT_BF16
+
+
+def test_unknown_names_and_sizes():
+    assert hip.kernel_choice("linear", 64, 64) is None
+    assert hip.kernel_choice("no such op", 64, 64, 64, 0) is None
+    assert hip.kernel_choice("linear", -1, 64, 64, 0) is None
+    assert hip.kernel_choice("linear", 0, 64, 64, 0) is None
+
+
+# rows, columns, K, flags: the fastest kernels
+LINEAR = [
+    # long K over some hundred rows: the K-split tiles read A and W once per
+    # 64 x 64 tile and lost to the 64-row tiles by 1.2 to 1.6 times
+    ((777, 1600, 6400, 0), {"db64x96", "db64x128"}),
+    ((1024, 1600, 6400, 0), {"db64x128"}),
+    ((1400, 896, 4864, 0), {"db64x96", "db64x128"}),
+    ((2048, 896, 4864, 0), {"db64x128"}),
+    ((777, 1600, 6400, ACT), {"db64x96", "db64x128"}),
+    ((1024, 1600, 6400, ACT), {"db64x128"}),
+    ((1400, 896, 4864, ACT), {"db64x96", "db64x128"}),
+    ((384, 4096, 12288, ACT), {"db64x128", "db64x96", "db64x64"}),
+    # bf16 activations halve the matrix work of a tile, not its reads
+    ((128, 50257, 1600, ACT), {"pp256x224", "pp256x256"}),
+    ((1024, 6144, 1024, ACT), {"db64x128"}),
+    ((33, 300, 200, 0), {"kw16x32"}),
+    # sizes that ran the right kernel before
+    ((97, 768, 3072, 0), {"kw16x32"}),
+    ((200, 2304, 768, 0), {"kw32x64"}),
+    ((512, 3072, 768, ACT), {"db64x96", "db64x128"}),
+    ((777, 4096, 1024, 0), {"db64x128"}),
+    ((777, 50257, 768, 0), {"pp256x160", "pp256x192", "pp256x224"}),
+    ((2048, 4800, 1600, 0), {"pp256x160", "pp256x192"}),
+    ((8192, 6400, 1600, 0), {"pp256x160", "pp256x192", "pp256x224"}),
+]
+
+
+@pytest.mark.parametrize("dims,names", LINEAR, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "")
+def test_linear_kernel(dims, names):
+    assert hip.kernel_choice("linear", *dims) in names
+
+
+@pytest.mark.parametrize("M,N,K", [(5_000_000, 16, 64), (6_000_000, 64, 8), (8_300_000, 8, 8), (300_000, 8, 8),
+                                   (4_400_000, 128, 512)])
+def test_linear_many_rows_fit_a_grid(M, N, K):
+    """A grid has at most 65,535 row tiles: sizes that 128-row tiles took (8.3
+    million rows) may not be sent to smaller ones."""
+    name = hip.kernel_choice("linear", M, N, K, 0)
+    rows = int(name.lstrip("dbkwp").split("x")[0])
+    assert -(-M // rows) <= 65535
+
+
+@pytest.mark.parametrize("M,N,K", [(4096, 4096, 1 << 21), (2048, 3 << 20, 64), (20000, 64, 5 << 19), (4096, 256, 1 << 21)])
+def test_linear_wide_rows_fit_a_resource(M, N, K):
+    """The rows of one tile (of A, and of a residual) stay below the 2 GiB of
+    a buffer resource, less the 64 KiB past its out-of-range offset."""
+    for flags in (0, ACT):
+        name = hip.kernel_choice("linear", M, N, K, flags)
+        rows = int(name.lstrip("dbkwp").split("x")[0])
+        assert rows * max(N, K) * 4 < 0x7FFF0000
