@@ -876,11 +876,23 @@ const char* gemm_choice_name(int M, int N, int K, bool act_bf16) {
 }
 
 // y[m, n] = silu(x W[n]) * (x W[N + n]) over a [2N, K] weight for more than 16
-// rows; false when the K-split tiles should take the product instead (few
-// tiles) or a weight panel spans 2 GiB.
+// rows: k_gemm_db's paired epilogue, where it is estimated faster than the
+// Linear of 2N columns and a SwiGLU launch. Both sides are fitted to 220
+// measured sizes (17 to 8,192 rows; the choice is on average 0.2% off the
+// faster side); the launch's 12 bytes an output mostly come from the Linear's
+// output still in cache. The K-split tiles keep few rows (17 x 1024 x 2 x 3072
+// 8.4 us against 12.4 paired) and the 256-row tiles long and wide prompts
+// (1400 x 2560 x 2 x 9728 278 against 320, 2048 x 4096 x 2 x 12288 690 / 924);
+// in between the pair wins (777 x 1024 x 2 x 3072 36.9 / 30.1, 8192 x 896 x 2 x
+// 4864 391 / 353).
 bool gemm_pair_swiglu_ok(int M, int N, int K) {
-    const GemmKind k = gemm_choice(M, 2 * N, K, false).kind;
-    return M > 16 && !(k >= kKw16x32 && k <= kKw64x64) && (long long)2 * N * K * 2 < (1ll << 31);
+    // the resource over the gate and the up rows; the grid's second dimension
+    if (M <= 16 || 4ll * N * K >= kOutOfRange || M > 64 * 65535) return false;
+    auto cdiv = [](long long a, long long b) { return (a + b - 1) / b; };
+    const double cus = cu_count(), out = 4e-6 * M * N, k = (double)cdiv(K, 64);
+    const double blocks = (double)cdiv(M, 64) * cdiv(N, 64), n = std::ceil(blocks / cus);
+    const double pair = 3.85 + k * (0.165 * std::ceil(n / 2) + 0.418 * n + 0.0344 * blocks / cus) + 0.329 * out;
+    return pair < gemm_choice(M, 2 * N, K, false).us + 2.3 + 0.571 * out;
 }
 int launch_gemm_pair_swiglu(hipStream_t s, const float* A, const uint16_t* W, float* y, int M, int N, int K) {
     const dim3 grid((N + 63) / 64, (M + 63) / 64);

@@ -17,7 +17,7 @@
 //   5. down GEMV with the residual add.
 // Longer inputs (prefill) take the same steps with the norms as launches of
 // their own and the matrix-core GEMMs for the Linears, SwiGLU in the gate/up
-// GEMM's epilogue.
+// GEMM's epilogue where that is the faster form.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -88,8 +88,8 @@ static int qwen_block_core(hipStream_t s, const gorch_hip_qwen_block* b, float* 
                                      GORCH_HIP_EPI_NONE, sw);
     }
     // longer inputs: h = RMSNorm_ffn(x1), the gate/up GEMM with SwiGLU in its
-    // epilogue, down; where that GEMM's tiles split K, gate and up as two
-    // column segments and a SwiGLU launch
+    // epilogue or, where another GEMM is faster by more than that saves, gate
+    // and up as two column segments and a SwiGLU launch; down
     GH_TRY(launch_rmsnorm(s, x1, b->norm_ffn, h, S, d, b->eps));
     if (gemm_pair_swiglu_ok(S, F, d)) {
         GH_TRY(launch_gemm_pair_swiglu(s, h, b->wgate_up, gu, S, F, d));

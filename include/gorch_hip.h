@@ -142,7 +142,9 @@ void gorch_hip_reset_dispatch_counts(void);
  * profiles: no device work, static strings, NULL for an unknown op or sizes
  * that launch nothing. op and dims:
  *   "linear" {M, N, K, flags}: gorch_hip_linear_bf16_ex above 16 rows (any
- *     number of rows with GORCH_HIP_LINEAR_ACT_BF16).
+ *     number of rows with GORCH_HIP_LINEAR_ACT_BF16);
+ *   "gate_up" {rows, inter, dim}: a Qwen block's gate/up product and SwiGLU
+ *     above 16 rows ("pair...": in one kernel).
  * The names are not an interface: they change with the kernels. */
 const char* gorch_hip_kernel_choice(const char* op, const int* dims, int n);
 

@@ -67,3 +67,25 @@ def test_linear_wide_rows_fit_a_resource(M, N, K):
         name = hip.kernel_choice("linear", M, N, K, flags)
         rows = int(name.lstrip("dbkwp").split("x")[0])
         assert rows * max(N, K) * 4 < 0x7FFF0000
+
+
+# rows, inter, dim: whether SwiGLU in the product's epilogue is the faster form
+GATE_UP = [
+    # long and wide prompts: the 256-row tiles and a SwiGLU launch were 1.1 to
+    # 1.4 times as fast as the paired 64-row tiles that ran
+    ((512, 12288, 4096), False), ((1400, 9728, 2560), False), ((2048, 12288, 4096), False), ((8192, 9728, 2560), False),
+    # a few rows of a wide weight: paired, the K-split tiles read it no faster
+    ((64, 12288, 4096), True), ((128, 3072, 1024), True),
+    # sizes that ran the right form before
+    ((17, 3072, 1024), False), ((777, 3072, 1024), True), ((1400, 4864, 896), True), ((4096, 1368, 512), True),
+]
+
+
+@pytest.mark.parametrize("dims,paired", GATE_UP, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "")
+def test_gate_up_form(dims, paired):
+    assert hip.kernel_choice("gate_up", *dims).startswith("pair") == paired
+
+
+def test_gate_up_limits():
+    """The pair's resource spans gate and up rows: 2 GiB at most."""
+    assert not hip.kernel_choice("gate_up", 64, 1 << 18, 2048).startswith("pair")
