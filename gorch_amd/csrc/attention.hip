@@ -15,6 +15,7 @@
 // P.V with lanes across the head's dims (coalesced 256-byte rows) and waves
 // across keys, the 4 wave partials summed in wave order.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -466,14 +467,15 @@ __global__ __launch_bounds__(NW * 64) void k_attn_rows(AttnArgs a) {
 // Bound by the f32 matrix cores (64 FLOP/clock and SIMD; 2.5 GFLOP at 777
 // rows of 16 heads of 128 take 18 us on all CUs) and by the longest chain:
 // a wave that walked all 777 keys for its 16 rows would take 46 us alone. So
-// a block of 8 waves takes 32 query rows (row group w & 1) and splits each
-// 64-key stage over 4 key groups (w >> 1), whose online softmax states are
+// a block of 8 waves takes 32 query rows (two row groups of 16) and splits
+// each 64-key stage over KG = 4 key groups, whose online softmax states are
 // merged in key-group order at the end; blocks go out longest first. With
-// an even number of query heads per KV head the two row groups are 16 rows
-// of two heads that share the staged keys. 777 rows, 16 / 8 heads of 128:
-// 160 us with 128 rows per block and no key groups, 45 us so; 16 x 512 rows,
-// 25 heads of 64: 330 -> 214 us (63 TFLOP/s; the softmax between the two
-// products is what the matrix cores wait for).
+// an even number of query heads per KV head the row groups are dealt to two
+// heads that share the staged keys. 777 rows, 16 / 8 heads of 128: 160 us
+// with 128 rows per block and no key groups, 45 us so; 16 x 512 rows, 25
+// heads of 64: 330 -> 214 us (63 TFLOP/s; the softmax between the two
+// products is what the matrix cores wait for). KG = 1 (128 rows, no merge) is
+// for many blocks over few keys (flash_key_groups).
 //
 // K and V stages go straight from the cache to LDS (raw buffer loads to LDS,
 // 16 bytes a lane, rows past the end zero), row-major, the stage after next
@@ -519,21 +521,24 @@ struct FlashStage {
     }
 };
 
-template <int HD>
+template <int HD, int KG>
 __global__ __launch_bounds__(512) void k_attn_flash(AttnArgs a, int heads, int pair) {
-    constexpr int QU = HD / 16;
+    constexpr int QU = HD / 16, RG = 8 / KG;
     // one array per stage, so that reads of one are known not to wait for
     // the loads into the other
     __shared__ __align__(16) float st0[FlashStage<HD>::kFloats];
     __shared__ __align__(16) float st1[FlashStage<HD>::kFloats];
-    __shared__ float red[2][4][2][16];  // [row group][key group][m, l][query]
+    __shared__ float red[KG > 1 ? RG : 1][KG][2][16];  // [row group][key group][m, l][query]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int rg = wave & 1, kg = wave >> 1, r = lane & 15, g = lane >> 4;
-    const int b = blockIdx.z, tile = gridDim.y - 1 - blockIdx.y;
-    // pair: rows of two heads of one KV head, else 32 rows of one head
-    const int h = pair ? 2 * (int)blockIdx.x + rg : (int)blockIdx.x;
-    const int q0 = pair ? tile * 16 : tile * 32 + rg * 16;  // the wave's first query row
-    const int qlast = min(a.new_seq, tile * (pair ? 16 : 32) + (pair ? 16 : 32)) - 1;
+    const int rg = wave % RG, kg = wave / RG, r = lane & 15, g = lane >> 4;
+    // blockIdx.x: row tile (longest first) times head or pair of heads
+    const int cols = pair ? heads / 2 : heads, b = blockIdx.z;
+    const int tile = gridDim.x / cols - 1 - blockIdx.x / cols, col = blockIdx.x % cols;
+    // pair: 8 RG rows of two heads of one KV head, else 16 RG rows of one head
+    const int h = pair ? 2 * col + (rg & 1) : col;
+    const int trows = pair ? 8 * RG : 16 * RG;
+    const int q0 = tile * trows + (pair ? rg >> 1 : rg) * 16;  // the wave's first query row
+    const int qlast = min(a.new_seq, tile * trows + trows) - 1;
     const int qi = q0 + r;                                   // this lane's query (column of S^T)
     const int pos = a.pos_dev ? *a.pos_dev : a.pos_host;
     const int kvh = a.kv_heads ? h / (heads / a.kv_heads) : h;
@@ -541,8 +546,8 @@ __global__ __launch_bounds__(512) void k_attn_flash(AttnArgs a, int heads, int p
     const size_t cbase = (size_t)b * a.max_seq * kvd + (size_t)__builtin_amdgcn_readfirstlane(kvh) * HD;
     const int t_all = pos + a.new_seq;
     const int kend = a.causal ? pos + qlast + 1 : t_all;
-    // the last key any of the wave's queries sees
-    const int kwave = a.causal ? min(t_all, pos + q0 + 16) : (q0 < a.new_seq ? t_all : 0);
+    // the keys any of the wave's queries sees (none past the last query)
+    const int kwave = q0 >= a.new_seq ? 0 : a.causal ? min(t_all, pos + q0 + 16) : t_all;
     const long long span = ((long long)(t_all - 1) * kvd + HD) * 4;
     const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.kc + cbase, span);
     const __amdgpu_buffer_rsrc_t rv = make_rsrc(a.vc + cbase, span);
@@ -560,9 +565,9 @@ __global__ __launch_bounds__(512) void k_attn_flash(AttnArgs a, int heads, int p
     for (int t = 0; t < QU; t++) o[t] = floatx4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;
 
-    auto slice = [&](const float* buf, int k0) {
-        const float* Ks = buf + (kg * 16 + r) * HD;
-        const int voff = (kFlashKeys + kg * 16 + 4 * g) * HD;
+    auto slice = [&](const float* buf, int k0, int ks) {
+        const float* Ks = buf + (ks * 16 + r) * HD;
+        const int voff = (kFlashKeys + ks * 16 + 4 * g) * HD;
         floatx4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int u = 0; u < QU; u++) {
@@ -576,7 +581,7 @@ __global__ __launch_bounds__(512) void k_attn_flash(AttnArgs a, int heads, int p
         float tmax = -INFINITY;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            const int key = k0 + kg * 16 + 4 * g + v;
+            const int key = k0 + ks * 16 + 4 * g + v;
             const bool ok = key < t_all && (!a.causal || key <= P);
             sv[v] = ok ? s[v] * a.scale : -INFINITY;
             tmax = fmaxf(tmax, sv[v]);
@@ -611,7 +616,9 @@ __global__ __launch_bounds__(512) void k_attn_flash(AttnArgs a, int heads, int p
     auto stage = [&](float* cur, float* nxt, int k0) {
         block_sync_dma();
         if (k0 + kFlashKeys < kend) FlashStage<HD>::issue(nxt, rk, rv, k0 + kFlashKeys, t_all, kvd);
-        if (k0 + kg * 16 < kwave) slice(cur, k0);
+#pragma unroll 1
+        for (int ks = kg; ks < 4; ks += KG)
+            if (k0 + ks * 16 < kwave) slice(cur, k0, ks);
     };
     for (int k0 = 0; k0 < kend; k0 += 2 * kFlashKeys) {
         stage(st0, st1, k0);
@@ -619,41 +626,51 @@ __global__ __launch_bounds__(512) void k_attn_flash(AttnArgs a, int heads, int p
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    // merge the 4 key groups: common maximum, then the rescaled sums
-    if (g == 0) {
-        red[rg][kg][0][r] = m;
-        red[rg][kg][1][r] = l;
-    }
-    __syncthreads();
-    float M = -INFINITY, L = 0.f;
+    const int orow = b * a.new_seq + qi;
+    if constexpr (KG == 1) {
+        if (!qok) return;
+        const float inv = 1.0f / l;
 #pragma unroll
-    for (int k = 0; k < 4; k++) M = fmaxf(M, red[rg][k][0][r]);
+        for (int t = 0; t < QU; t++)
+            attn_out4(a, orow, h * HD + 16 * t + 4 * g,
+                      make_float4(o[t][0] * inv, o[t][1] * inv, o[t][2] * inv, o[t][3] * inv));
+    } else {
+        // merge the key groups: common maximum, then the rescaled sums
+        if (g == 0) {
+            red[rg][kg][0][r] = m;
+            red[rg][kg][1][r] = l;
+        }
+        __syncthreads();
+        float M = -INFINITY, L = 0.f;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const float mk = red[rg][k][0][r];
-        L += mk == -INFINITY ? 0.f : red[rg][k][1][r] * expf(mk - M);
-    }
-    const float sc = m == -INFINITY ? 0.f : expf(m - M);
-    // (every wave has left the stages: the barrier above)
-    float4* mo = reinterpret_cast<float4*>(st0);  // [row group][key group][t][lane]
-    static_assert(8 * QU * 64 * 4 <= FlashStage<HD>::kFloats, "merge buffer");
+        for (int k = 0; k < KG; k++) M = fmaxf(M, red[rg][k][0][r]);
 #pragma unroll
-    for (int t = 0; t < QU; t++)
-        mo[((rg * 4 + kg) * QU + t) * 64 + lane] = make_float4(o[t][0] * sc, o[t][1] * sc, o[t][2] * sc, o[t][3] * sc);
-    __syncthreads();
-    if (qok) {
-        const int orow = b * a.new_seq + qi;
-        const float inv = 1.0f / L;
+        for (int k = 0; k < KG; k++) {
+            const float mk = red[rg][k][0][r];
+            L += mk == -INFINITY ? 0.f : red[rg][k][1][r] * expf(mk - M);
+        }
+        const float sc = m == -INFINITY ? 0.f : expf(m - M);
+        // (every wave has left the stages: the barrier above)
+        float4* mo = reinterpret_cast<float4*>(st0);  // [row group][key group][t][lane]
+        static_assert(8 * QU * 64 * 4 <= FlashStage<HD>::kFloats, "merge buffer");
 #pragma unroll
-        for (int tt = 0; tt < QU / 4; tt++) {
-            const int t = kg * (QU / 4) + tt;
-            float4 s = mo[(rg * 4 * QU + t) * 64 + lane];
+        for (int t = 0; t < QU; t++)
+            mo[((rg * KG + kg) * QU + t) * 64 + lane] =
+                make_float4(o[t][0] * sc, o[t][1] * sc, o[t][2] * sc, o[t][3] * sc);
+        __syncthreads();
+        if (qok) {
+            const float inv = 1.0f / L;
 #pragma unroll
-            for (int k = 1; k < 4; k++) {
-                const float4 v = mo[((rg * 4 + k) * QU + t) * 64 + lane];
-                s = make_float4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w);
+            for (int tt = 0; tt < QU / KG; tt++) {
+                const int t = kg * (QU / KG) + tt;
+                float4 s = mo[(rg * KG * QU + t) * 64 + lane];
+#pragma unroll
+                for (int k = 1; k < KG; k++) {
+                    const float4 v = mo[((rg * KG + k) * QU + t) * 64 + lane];
+                    s = make_float4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w);
+                }
+                attn_out4(a, orow, h * HD + 16 * t + 4 * g, make_float4(s.x * inv, s.y * inv, s.z * inv, s.w * inv));
             }
-            attn_out4(a, orow, h * HD + 16 * t + 4 * g, make_float4(s.x * inv, s.y * inv, s.z * inv, s.w * inv));
         }
     }
 }
@@ -1140,6 +1157,9 @@ static int attn_split_chunks(const AttnArgs& a, int heads, int rows) {
 // sequence, the (key, chunk)-lane kernel for short caches, the online-softmax
 // kernel for few (head, row) blocks over a long cache, else the two-pass
 // cached kernel (16 waves when blocks are few and the cache long).
+// Query heads of a KV head in pairs: the prefill kernel's blocks take two.
+static bool flash_pairs(const AttnArgs& a, int heads) { return a.kv_heads && (heads / a.kv_heads) % 2 == 0; }
+
 static AttnRoute attn_route(const AttnArgs& a, int heads, int rows) {
     // the score-staging kernels hold one f32 per visible key in LDS: at most
     // the cache capacity when the cache length is read on the device, else
@@ -1154,7 +1174,19 @@ static AttnRoute attn_route(const AttnArgs& a, int heads, int rows) {
     // of 5, 2000 blocks, 505 keys 31.8 / 75.8; but 4 of 4, 400 blocks 7.5 /
     // 6.8, and 20 rows of one sequence of 16 heads over 1020 keys, 320
     // blocks, 50 / 22.5: few rows leave most of a 32-row tile empty).
-    const bool many_rows = a.new_seq >= 32 || (a.new_seq >= 4 && blocks >= 1536);
+    bool many_rows = a.new_seq >= 32 || (a.new_seq >= 4 && blocks >= 1536);
+    // Fewer than 8 rows where an odd number of query heads shares a KV head of
+    // 128: the other kernels find K and V in L2, so the prefill kernel's
+    // rounds (a block per head and sequence, one a CU) have to hold 4 times as
+    // many rows as CUs (28 heads on 4, 504 keys: 14 sequences of 4 rows, 55.0
+    // against 43.2; 11 of 5 54.2 / 41.6; 20 of 6 80.4 / 80.4; 904 keys 137 /
+    // 161); up to 256 keys one 8-wave block per row is slower still (239 keys,
+    // 14 of 4, 32.4 / 56.2).
+    if (many_rows && a.new_seq < 8 && a.hd == 128 && a.kv_heads && a.kv_heads != heads && !flash_pairs(a, heads) &&
+        (a.max_seq <= 128 || a.max_seq > 256)) {
+        const int rounds = (heads * (rows / a.new_seq) + 255) / 256;
+        many_rows = 1024 * rounds <= blocks;
+    }
     const bool aligned = (a.q_stride % 4 == 0) && (a.dim % 4 == 0) && ((a.kv_dim ? a.kv_dim : a.dim) % 4 == 0) &&
                          ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.kc) |
                            reinterpret_cast<uintptr_t>(a.vc) | reinterpret_cast<uintptr_t>(a.out)) % 16 == 0);
@@ -1173,6 +1205,47 @@ static AttnRoute attn_route(const AttnArgs& a, int heads, int rows) {
     // 29.4 us per layer)
     if (aligned && (blocks < 128 || !lds_ok) && (a.hd == 64 || a.hd == 128)) return kRouteLong;
     return cached();
+}
+
+// Key groups of the matrix-core prefill kernel: 4, or 1 when the 4-group form
+// needs several rounds of blocks (two blocks fit a CU at head dim 64, one at
+// 128) that gain nothing by splitting keys, each with its own merge:
+//   up to three 64-key stages in all: 16 x 128 rows, 32 / 8 heads of 128 68 us
+//     against 57 with one group, 37 keys before them 90 / 75 (the kernel
+//     without key groups this replaced 57 / 79); 16 x 40 rows, 25 heads of 64
+//     13.3 / 9.5; but in one round 8 x 64 rows, 8 heads of 128 7.3 / 11.5;
+//   head dim 128, paired heads and mostly cached keys, whose tiles of rows all
+//     end near the same key: 16 x 128 rows after 500, 32 / 8 heads 257 / 242,
+//     16 / 8 heads 138 / 125.
+// Otherwise the shorter 4-group blocks even out better: 4 x 777 rows, 25 heads
+// of 64 115 / 171.
+static int flash_key_groups(const AttnArgs& a, int heads, int batch, bool pair) {
+    const int rows1 = pair ? 64 : 128;  // query rows of a block with one group
+    const long long cols = (long long)(pair ? heads / 2 : heads) * batch;
+    const long long blocks4 = cols * ((a.new_seq + rows1 / 4 - 1) / (rows1 / 4));
+    const long long keys = (long long)a.pos_host + a.new_seq;
+    if (a.pos_dev || a.new_seq < 32) return 4;
+    if (keys <= 3 * kFlashKeys && blocks4 > (a.hd == 64 ? 512 : 640)) return 1;
+    const int last = a.new_seq % rows1;
+    if (a.hd == 128 && pair && blocks4 >= 768 && a.pos_host >= 3 * a.new_seq && (last == 0 || last >= rows1 * 7 / 8)) return 1;
+    return 4;
+}
+
+// The route's name for a causal call over 16-byte aligned buffers
+// (gorch_hip_kernel_choice).
+const char* attn_choice_name(int batch, int new_seq, int pos, int heads, int kv_heads, int hd, int max_seq) {
+    const int kvd = (kv_heads ? kv_heads : heads) * hd;
+    const AttnArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, pos, new_seq, heads * hd, hd, max_seq, heads * hd, 1,
+                     1.f, kv_heads, kvd, 1};
+    switch (attn_route(a, heads, batch * new_seq)) {
+        case kRouteFlash: return flash_key_groups(a, heads, batch, flash_pairs(a, heads)) == 1 ? "prefill_kg1" : "prefill_kg4";
+        case kRouteSplit: return "split";
+        case kRouteRows: return "rows";
+        case kRouteLong: return "long";
+        case kRouteCached16: return "cached16";
+        case kRouteCached4: return "cached4";
+        default: return nullptr;
+    }
 }
 
 bool attn_rows_wo_ok(const AttnArgs& a, int heads, int rows) {
@@ -1233,10 +1306,19 @@ int launch_attn_cached(hipStream_t s, const AttnArgs& a, int heads, int rows) {
         case kRouteFlash: {
             // many new rows per sequence (prefill): the matrix-core kernel
             const int batch = rows / a.new_seq;
-            const int pair = a.kv_heads && (heads / a.kv_heads) % 2 == 0;
-            const dim3 fg(pair ? heads / 2 : heads, pair ? (a.new_seq + 15) / 16 : (a.new_seq + 31) / 32, batch);
-            if (a.hd == 64) hipLaunchKernelGGL((k_attn_flash<64>), fg, dim3(512), 0, s, a, heads, pair);
-            else hipLaunchKernelGGL((k_attn_flash<128>), fg, dim3(512), 0, s, a, heads, pair);
+            const bool pair = flash_pairs(a, heads);
+            const auto launch = [&](auto hd, auto kg) {
+                constexpr int HD = decltype(hd)::value, KG = decltype(kg)::value;
+                const int trows = pair ? 64 / KG : 128 / KG;
+                const dim3 fg((pair ? heads / 2 : heads) * ((a.new_seq + trows - 1) / trows), 1, batch);
+                hipLaunchKernelGGL((k_attn_flash<HD, KG>), fg, dim3(512), 0, s, a, heads, pair);
+            };
+            const auto groups = [&](auto hd) {
+                if (flash_key_groups(a, heads, batch, pair) == 1) launch(hd, std::integral_constant<int, 1>{});
+                else launch(hd, std::integral_constant<int, 4>{});
+            };
+            if (a.hd == 64) groups(std::integral_constant<int, 64>{});
+            else groups(std::integral_constant<int, 128>{});
             count(CNT_ATTENTION);
             return check_launch("attn_flash");
         }

@@ -144,7 +144,10 @@ void gorch_hip_reset_dispatch_counts(void);
  *   "linear" {M, N, K, flags}: gorch_hip_linear_bf16_ex above 16 rows (any
  *     number of rows with GORCH_HIP_LINEAR_ACT_BF16);
  *   "gate_up" {rows, inter, dim}: a Qwen block's gate/up product and SwiGLU
- *     above 16 rows ("pair...": in one kernel).
+ *     above 16 rows ("pair...": in one kernel);
+ *   "attention" {batch, new rows, cached rows, heads, KV heads (0: one per
+ *     head), head_dim, max_seq}: a causal attention_cached call over 16-byte
+ *     aligned buffers.
  * The names are not an interface: they change with the kernels. */
 const char* gorch_hip_kernel_choice(const char* op, const int* dims, int n);
 

@@ -1,7 +1,8 @@
 """The prefill attention kernel at the edges of its tiles: rows around the
 16- and 32-row groups, keys around the 64-key stages and 16-key groups, paired
-and unpaired query heads, causal and not, few rows of many sequences, and
-NaNs in the cache rows past the last key.
+and unpaired query heads, causal and not, few rows of many sequences, NaNs in the
+cache rows past the last key; the form without key groups (128 rows a block,
+or 64 of two heads) at the edges of its own tiles.
 
 Bound: float64 attention over the same inputs, 1e-6 in the 2-norm (f32
 products and sums over up to 700 keys measure 2-4e-7; probabilities rounded
@@ -22,9 +23,20 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
-def test_flash_tiles(gpu, case):
+ONE_GROUP = [
+    (24, 33, 0, 14, 2, 64, 1), (24, 33, 0, 14, 2, 64, 0), (5, 129, 60, 25, 25, 64, 1), (12, 40, 5, 32, 16, 64, 1),
+    (12, 65, 127, 32, 16, 64, 0), (30, 33, 100, 12, 12, 128, 1), (7, 145, 47, 19, 19, 128, 1), (14, 47, 17, 32, 8, 128, 1),
+    (14, 64, 128, 32, 8, 128, 0),
+    # mostly cached keys, past three stages
+    (12, 57, 180, 32, 8, 128, 1), (12, 64, 321, 32, 8, 128, 0),
+]
+
+
+@pytest.mark.parametrize("case,name", [(c, "prefill_kg4") for c in CASES] + [(c, "prefill_kg1") for c in ONE_GROUP],
+                         ids=lambda c: "x".join(map(str, c)) if isinstance(c, tuple) else c)
+def test_flash_tiles(gpu, case, name):
     B, n, pos, hq, hkv, hd, causal = case
+    assert gpu.kernel_choice("attention", B, n, pos, hq, hkv, hd, pos + n + 5) == name
     rng = np.random.default_rng(n + pos + hq)
     T, cap = pos + n, pos + n + 5
     q = rng.standard_normal((B, n, hq, hd)).astype(np.float32)

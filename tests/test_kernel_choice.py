@@ -89,3 +89,25 @@ def test_gate_up_form(dims, paired):
 def test_gate_up_limits():
     """The pair's resource spans gate and up rows: 2 GiB at most."""
     assert not hip.kernel_choice("gate_up", 64, 1 << 18, 2048).startswith("pair")
+
+
+# batch, new rows, cached rows, heads, KV heads, head_dim, max_seq
+ATTENTION = [
+    # several rounds of 32-row blocks over few keys, each with a merge of its
+    # own: 1.06 to 1.2 times the time of the kernel without key groups before
+    ((16, 128, 0, 32, 8, 128, 136), {"prefill_kg1"}), ((16, 100, 37, 16, 8, 128, 145), {"prefill_kg1"}),
+    ((16, 128, 500, 32, 8, 128, 636), {"prefill_kg1"}), ((16, 40, 0, 25, 25, 64, 48), {"prefill_kg1"}),
+    # few rows of an odd group of 128-wide heads: 1.2 to 1.3 times the time of
+    # the kernels with a block per row
+    ((14, 4, 500, 28, 4, 128, 504), {"cached4"}), ((11, 5, 500, 28, 4, 128, 505), {"cached4"}),
+    # the right ones before
+    ((14, 8, 500, 28, 4, 128, 508), {"prefill_kg4"}), ((22, 5, 235, 28, 4, 128, 240), {"prefill_kg4"}),
+    ((1, 777, 0, 16, 8, 128, 1024), {"prefill_kg4"}), ((16, 512, 0, 25, 25, 64, 512), {"prefill_kg4"}),
+    ((8, 64, 0, 8, 8, 128, 72), {"prefill_kg4"}), ((4, 777, 37, 25, 25, 64, 814), {"prefill_kg4"}),
+    ((16, 1, 640, 25, 0, 64, 768), {"cached16"}), ((1, 20, 1000, 16, 8, 128, 1020), {"cached16"}),
+]
+
+
+@pytest.mark.parametrize("dims,names", ATTENTION, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "")
+def test_attention_kernel(dims, names):
+    assert hip.kernel_choice("attention", *dims) in names
