@@ -73,17 +73,20 @@ struct MmOperand {
         const int tid = threadIdx.x & 255;
         return 8 * (KC ? (tid + 256 * i) % CH : tid / (T / P));
     }
-    // element loads of a ragged step: zeros past K, rows clamped into the matrix
-    template <bool KC>
+    // element loads of a ragged step: zeros past K; rows past the last one are
+    // clamped to it, or with SKIP read as zeros too, which costs a compare but
+    // no memory traffic (thin outputs: 263 x 1547 x 1 x 28 hh 14.7 -> 12.0 us;
+    // but 39 x 29 x 1093 x 80 hh, two steps, 7.1 -> 9.1)
+    template <bool KC, bool SKIP>
     __device__ static __forceinline__ void load_edge(const char* base, int r0, int R, int K, int k0, Patch& p) {
         const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, (long long)R * K * E);
 #pragma unroll
         for (int i = 0; i < P; i++) {
-            const int row = min(r0 + row_of<KC>(i), R - 1);
+            const int row = SKIP ? r0 + row_of<KC>(i) : min(r0 + row_of<KC>(i), R - 1);
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const int k = k0 + k_of<KC>(i) + e;
-                const int off = k < K ? (KC ? row * K + k : k * R + row) * E : kOutOfRange;
+                const int off = k < K && (!SKIP || row < R) ? (KC ? row * K + k : k * R + row) * E : kOutOfRange;
                 if constexpr (F32) {
                     p.w[i][e] = __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0);
                 } else {
@@ -181,15 +184,20 @@ struct MmOperand {
 // KA / KB: A stored [M][K] (not transA), B stored [N][K] (transB). G groups
 // of 4 waves share a block's tile: group q takes steps q, q + G, ... through
 // LDS stages of its own and the groups' sums are added in order at the end.
-template <int T, int G, int BK, bool KA, bool FA, bool KB, bool FB>
-__global__ __launch_bounds__(256 * G, G <= 2 ? 2 : 1) void k_mm(const void* __restrict__ A, const void* __restrict__ B,
+// ONE: the whole of K is one step (K <= BK). No second stage and no loop, so
+// that three to eight blocks fit a CU: such products are bound by their output,
+// and their tiles' loads, barriers and stores overlap only across blocks. They are
+// formed as A x B, one 4-byte column a lane: 16-byte stores of 16 rows at once
+// wrote 8192 x 8192 x 8 hh in 63 us, this in 52.
+template <int T, int G, int BK, bool KA, bool FA, bool KB, bool FB, bool ONE = false>
+__global__ __launch_bounds__(256 * G, ONE && BK == 32 ? 4 : G <= 2 ? 2 : 1) void k_mm(const void* __restrict__ A, const void* __restrict__ B,
                                                    float* __restrict__ C, int M, int N, int K, int xcd_map) {
     using OA = MmOperand<T, BK, FA>;
     using OB = MmOperand<T, BK, FB>;
     constexpr int TF = T / 32;  // 16-wide fragments per wave and side
     constexpr int STAGE = OA::ELEMS + OB::ELEMS;
     // two LDS stages (one barrier per step) while two blocks still fit a CU
-    constexpr int NS = 2 * G * STAGE * 2 <= (G > 1 ? 144 : 80) * 1024 ? 2 : 1;
+    constexpr int NS = !ONE && 2 * G * STAGE * 2 <= (G > 1 ? 144 : 80) * 1024 ? 2 : 1;
     constexpr size_t kRed = G > 1 ? (size_t)(G - 1) * T * T * 4 : 0;
     constexpr size_t kLds = (size_t)G * NS * STAGE * 2 > kRed ? (size_t)G * NS * STAGE * 2 : kRed;
     __shared__ __align__(16) char smem[kLds];
@@ -249,7 +257,9 @@ __global__ __launch_bounds__(256 * G, G <= 2 ? 2 : 1) void k_mm(const void* __re
                     for (int tb = 0; tb < OB::NT; tb++)
                         if (ta + tb <= 2)
 #pragma unroll
-                            for (int i = 0; i < TF; i++) acc[i][j] = mfma16x16x32(bfr[tb], af[i][ta], acc[i][j]);
+                            for (int i = 0; i < TF; i++)
+                                acc[i][j] = ONE ? mfma16x16x32(af[i][ta], bfr[tb], acc[i][j])
+                                                : mfma16x16x32(bfr[tb], af[i][ta], acc[i][j]);
             }
         }
     };
@@ -270,11 +280,29 @@ __global__ __launch_bounds__(256 * G, G <= 2 ? 2 : 1) void k_mm(const void* __re
             OA::template load<KA>(Ab, m0, M, K, s * BK, pa);
             OB::template load<KB>(Bb, n0, N, K, s * BK, pb);
         } else if (s < ns) {
-            OA::template load_edge<KA>(Ab, m0, M, K, s * BK, pa);
-            OB::template load_edge<KB>(Bb, n0, N, K, s * BK, pb);
+            OA::template load_edge<KA, ONE>(Ab, m0, M, K, s * BK, pa);
+            OB::template load_edge<KB, ONE>(Bb, n0, N, K, s * BK, pb);
         }
     };
+    float* Cb = C + (size_t)bz * M * N;
     load(grp);
+    if constexpr (ONE) {
+        static_assert(G == 1, "one step");
+        store(lds);
+        __syncthreads();
+        compute(lds);
+        // lane (r, g): column r, rows 4g .. 4g + 3 of each 16 x 16 fragment
+#pragma unroll
+        for (int i = 0; i < TF; i++)
+#pragma unroll
+            for (int j = 0; j < TF; j++) {
+                const int m = m0 + wm * (T / 2) + 16 * i + 4 * g, n = n0 + wn * (T / 2) + 16 * j + r;
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (m + v < M && n < N) Cb[(size_t)(m + v) * N + n] = acc[i][j][v];
+            }
+        return;
+    }
     if constexpr (NS == 2) {
         if (grp < ns) store(lds);
         __syncthreads();
@@ -318,7 +346,6 @@ __global__ __launch_bounds__(256 * G, G <= 2 ? 2 : 1) void k_mm(const void* __re
                 }
     }
     // lane (r, g): row r, columns 4g .. 4g + 3 of each 16 x 16 fragment
-    float* Cb = C + (size_t)bz * M * N;
 #pragma unroll
     for (int i = 0; i < TF; i++) {
         const int m = m0 + wm * (T / 2) + 16 * i + r;
@@ -339,15 +366,17 @@ __global__ __launch_bounds__(256 * G, G <= 2 ? 2 : 1) void k_mm(const void* __re
     }
 }
 
+// Tile, K groups and step width (BK; 0: 64, 32 for 128 x 128 tiles of f32).
 // HALF: two bf16 operands only (4 groups of 64 x 64 stages fit LDS then).
-template <int T, int G, bool HALF = false>
+template <int T, int G, int BK = 0, bool ONE = false, bool HALF = false>
 static void launch_mm_t(hipStream_t s, const void* A, const void* B, float* C, int M, int N, int K, int batch,
                         bool ka, bool fa, bool kb, bool fb) {
     const unsigned gx = (N + T - 1) / T, gy = (M + T - 1) / T;
     const int xcd_map = batch > 1 && (long long)gx * gy * batch < (1ll << 22);
     const dim3 grid = xcd_map ? dim3(gx * gy * batch) : dim3(gx, gy, batch);
-#define GH_MM(KA, FA, KB, FB) \
-    hipLaunchKernelGGL((k_mm<T, G, T == 128 && (FA || FB) ? 32 : 64, KA, FA, KB, FB>), grid, dim3(256 * G), 0, s, A, B, C, M, N, K, xcd_map)
+#define GH_MM(KA, FA, KB, FB)                                                                                      \
+    hipLaunchKernelGGL((k_mm<T, G, BK ? BK : (T == 128 && (FA || FB) ? 32 : 64), KA, FA, KB, FB, ONE>), grid, dim3(256 * G), \
+                       0, s, A, B, C, M, N, K, xcd_map)
 #define GH_MM_T(KA, KB)                              \
     do {                                             \
         if constexpr (HALF) GH_MM(KA, false, KB, false); \
@@ -376,17 +405,55 @@ static void launch_mm_t(hipStream_t s, const void* A, const void* B, float* C, i
 //     30 x 92 x 725 x 687 ff 41.7 / 50.3 / 50.9.
 //   128 x 128 from 512 such tiles: half the operand traffic, 4096^3 hh 165
 //     against 224 (64/1), fh 398 / 598; 48 x 512 x 512 x 64 ff 20.2 / 20.6.
-// The element-wise gather kernel this replaced: 1024^3 hh 52.4, 48 x 512 x
-// 512 x 64 ff 49.2.
-static void launch_mm(hipStream_t s, const void* A, const void* B, float* C, int M, int N, int K, int batch, bool ka,
-                      bool fa, bool kb, bool fb) {
+// Up to 64 deep a product is one step (ONE), of 32 up to 32: 192 x 1 x 640 x
+// 64 hh 5.1 us, 8.0 in 128 x 128 tiles; 54 x 1869 x 10 x 4 hh 5.4 / 12.8; 16 x
+// 16 x 16 3.4, 3.6 on four groups. 128 x 128 tiles stay where they are mostly
+// full (three 64 x 64 tiles in each at least) and
+//   K > 32: 48 x 1024 x 1024 x 40 ff 0.75 of the time of ONE;
+//   K 8 .. 32, 4096 tiles and more: 25 x 1753 x 1946 x 19 fh 90.4 / 123.8 (rows
+//     that start off a 64-byte line), 16 x 2048 x 2048 x 8 hh 57.6 / 63.0; but
+//     K = 4 8192 x 8192 54 / 43, and below 4096 tiles ONE is even or better
+//     (64 x 512 x 512 x 19 fh 18.7 / 17.3).
+// The element-wise gather kernel all this replaced: 1024^3 hh 52.4, 48 x 512 x
+// 512 x 64 ff 49.2; at 32 deep and less it had 32-wide steps and one stage, and
+// the sizes above took 8.5, 5.5, 3.4, 131 and 57 us.
+enum MmKind { kMm32x4, kMm64x4, kMm64x2, kMm64x1, kMm128, kMmOne32, kMmOne64, kMmOne64K64, kMm128K32 };
+static MmKind mm_kind(int M, int N, int K, int batch, bool half) {
     const long long n64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * batch;
     const long long n128 = (long long)((M + 127) / 128) * ((N + 127) / 128) * batch;
-    if (n64 <= 64) launch_mm_t<32, 4>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
-    else if (n64 <= 256 && !fa && !fb && K >= 512) launch_mm_t<64, 4, true>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
-    else if (n64 <= 256) launch_mm_t<64, 2>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
-    else if (n128 < 512) launch_mm_t<64, 1>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
-    else launch_mm_t<128, 1>(s, A, B, C, M, N, K, batch, ka, fa, kb, fb);
+    const bool full128 = n64 >= 3 * n128;
+    if (K <= 32) {
+        if (n128 >= 4096 && full128 && K >= 8) return kMm128K32;
+        return n64 <= 64 ? kMmOne32 : kMmOne64;
+    }
+    if (K <= 64 && (n128 < 512 || !full128)) return n64 <= 64 ? kMmOne32 : kMmOne64K64;
+    if (n64 <= 64) return kMm32x4;
+    if (n64 <= 256) return half && K >= 512 ? kMm64x4 : kMm64x2;
+    return n128 < 512 ? kMm64x1 : kMm128;
+}
+
+// The kernel's name (gorch_hip_kernel_choice).
+const char* matmul_choice_name(int M, int N, int K, int batch, bool a_bf16, bool b_bf16) {
+    static const char* const kName[] = {"mm32x4",  "mm64x4",  "mm64x2",     "mm64x1",    "mm128",
+                                        "mm32one", "mm64one", "mm64one_k64", "mm128_k32"};
+    return kName[mm_kind(M, N, K, batch, a_bf16 && b_bf16)];
+}
+
+static void launch_mm(hipStream_t s, const void* A, const void* B, float* C, int M, int N, int K, int batch, bool ka,
+                      bool fa, bool kb, bool fb) {
+#define GH_ARGS s, A, B, C, M, N, K, batch, ka, fa, kb, fb
+    switch (mm_kind(M, N, K, batch, !fa && !fb)) {
+        case kMm32x4: launch_mm_t<32, 4>(GH_ARGS); break;
+        case kMm64x4: launch_mm_t<64, 4, 0, false, true>(GH_ARGS); break;
+        case kMm64x2: launch_mm_t<64, 2>(GH_ARGS); break;
+        case kMm64x1: launch_mm_t<64, 1>(GH_ARGS); break;
+        case kMmOne32: launch_mm_t<32, 1, 64, true>(GH_ARGS); break;
+        case kMmOne64: launch_mm_t<64, 1, 32, true>(GH_ARGS); break;
+        case kMmOne64K64: launch_mm_t<64, 1, 64, true>(GH_ARGS); break;
+        case kMm128K32: launch_mm_t<128, 1, 32>(GH_ARGS); break;
+        default: launch_mm_t<128, 1>(GH_ARGS); break;
+    }
+#undef GH_ARGS
 }
 
 static bool linear_fast_ok(const void* x, const void* W, int K) {

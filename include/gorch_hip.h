@@ -145,6 +145,8 @@ void gorch_hip_reset_dispatch_counts(void);
  *     number of rows with GORCH_HIP_LINEAR_ACT_BF16);
  *   "gate_up" {rows, inter, dim}: a Qwen block's gate/up product and SwiGLU
  *     above 16 rows ("pair...": in one kernel);
+ *   "matmul" {M, N, K, batch, aBF16, bBF16}: the general product
+ *     (gorch_hip_matmul_dt's route to the Linear aside);
  *   "attention" {batch, new rows, cached rows, heads, KV heads (0: one per
  *     head), head_dim, max_seq}: a causal attention_cached call over 16-byte
  *     aligned buffers.

@@ -111,3 +111,22 @@ ATTENTION = [
 @pytest.mark.parametrize("dims,names", ATTENTION, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "")
 def test_attention_kernel(dims, names):
     assert hip.kernel_choice("attention", *dims) in names
+
+
+# M, N, K, batch, bf16 operands
+MATMUL = [
+    # small K and thin outputs: 128 x 128 tiles and 64-wide steps of mostly
+    # absent elements took 1.1 to 3 times the time of the kernel before them
+    ((1, 640, 64, 192, 1, 1), "mm64one_k64"), ((1547, 1, 28, 263, 1, 1), "mm64one"), ((1869, 10, 4, 54, 1, 1), "mm64one"),
+    ((836, 11, 9, 8, 1, 1), "mm64one"), ((36, 1351, 2, 91, 1, 1), "mm64one"), ((16, 16, 16, 1, 0, 0), "mm32one"),
+    ((512, 512, 16, 64, 1, 1), "mm64one"), ((2048, 2048, 8, 16, 1, 1), "mm128_k32"),
+    # the right ones before
+    ((512, 512, 64, 48, 0, 0), "mm128"), ((1753, 1946, 19, 25, 0, 1), "mm128_k32"), ((1024, 1024, 1024, 1, 1, 1), "mm64x4"),
+    ((1024, 1024, 1024, 1, 0, 0), "mm64x2"), ((2048, 2048, 2048, 1, 1, 1), "mm64x1"), ((4096, 4096, 4096, 1, 1, 1), "mm128"),
+    ((64, 64, 2048, 1, 0, 0), "mm32x4"),
+]
+
+
+@pytest.mark.parametrize("dims,name", MATMUL, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v)
+def test_matmul_kernel(dims, name):
+    assert hip.kernel_choice("matmul", *dims) == name
