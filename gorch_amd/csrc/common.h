@@ -404,6 +404,7 @@ bool gemv_pair_swiglu_ok(int F, int K);
 bool gemm_pair_swiglu_ok(int M, int N, int K);
 // Names for gorch_hip_kernel_choice.
 const char* gemm_choice_name(int M, int N, int K, bool act_bf16);
+const char* moe_choice_name(int tokens, int dim, int ffn, int experts, int top_k, bool down);
 const char* matmul_choice_name(int M, int N, int K, int batch, bool a_bf16, bool b_bf16);
 const char* attn_choice_name(int batch, int new_seq, int pos, int heads, int kv_heads, int hd, int max_seq);
 int launch_gemm_pair_swiglu(hipStream_t s, const float* x, const uint16_t* W, float* y, int M, int N, int K);

@@ -18,7 +18,8 @@
 //                    applied in the epilogue (the reference's Mul);
 //   k_moe_combine    out[t] = sum of the token's rows in ascending expert order.
 // Decode batches run router, top-K and routing in one launch (k_moe_front),
-// and few rows per expert take K-split tiles (k_moe_kw) in either grouped GEMM.
+// and layers of few row tiles take K-split tiles (k_moe_kw) in either grouped
+// GEMM (moe_tiles).
 // Expert weights are stacked [E][out][in] bf16 in one device array each.
 #include <algorithm>
 
@@ -422,16 +423,14 @@ __global__ __launch_bounds__(1024) void k_moe_front(const float* __restrict__ x,
     }
 }
 
-// out[t] = sum over the token's K packed rows in ascending expert order
-// (the reference adds each expert's ScatterAdd contribution in order). One
-// thread per (token, 4 columns); dim % 4 == 0. nsl > 1: the down GEMM left
-// raw K-slice partials, and a row's value is ((sum of slices) + bias) * w.
 // out[t] = the token's K expert rows summed in ascending expert order
-// (nn/moe.go:155-180). KT >= K slots: the token's expert indices and packed
-// rows are loaded together, sorted in registers, then every row's chunk is
-// loaded at once (raw buffer loads, unused slots out of range), so a chunk
-// costs two dependent round trips. With nsl > 1 K slices of the down GEMM
-// the slices, bias and routing weight are added here.
+// (nn/moe.go:155-180: each expert's ScatterAdd contribution in order). One
+// thread per (token, 4 columns); dim % 4 == 0. KT >= K slots: the token's
+// expert indices and packed rows are loaded together, sorted in registers,
+// then every row's chunk is loaded at once (raw buffer loads, unused slots out
+// of range), so a chunk costs two dependent round trips. nsl > 1: the down
+// GEMM left raw K-slice partials, and a row's value is ((sum of slices) +
+// bias) * w.
 template <int KT>
 __global__ void k_moe_combine(const float* __restrict__ yg, const int* __restrict__ inv,
                               const int* __restrict__ topi, float* out, int M, int K, int dim, int nsl,
@@ -512,9 +511,8 @@ __global__ void k_moe_combine(const float* __restrict__ yg, const int* __restric
 // Wide-tile path. The gather writes Xg as two bf16 planes (hi, lo: x = hi +
 // lo to ~2^-16 relative, the split the MFMA kernels use) in the space of the
 // f32 Xg, and GEMM 1's epilogue writes H the same way, so both GEMMs load
-// 16-byte bf16 words only. Rows are grouped in 128-row tiles. The down GEMM
-// takes 256-wide tiles where 128-wide ones would need a second round of CUs
-// (2048 tokens at d = 1024: 97 us on 144 blocks, 113 on 288).
+// 16-byte bf16 words only. Rows are grouped in 128-row tiles (column widths:
+// moe_tiles).
 // Splitting the down GEMM's K over twice the blocks (raw partials, summed
 // with bias and routing weight by the combine) measured within noise of the
 // unsplit kernel (118 vs 121 us): these GEMMs are bound by the traffic from
@@ -896,6 +894,56 @@ __global__ __launch_bounds__(64 * G) void k_moe_kw(const uint16_t* __restrict__ 
     }
 }
 
+// Tiles of the two expert GEMMs, by the row tiles that can be live (one per
+// expert reached and one more per 128 rows) and the rows an expert has on
+// average. The K-split tiles (k_moe_kw) read a weight panel once per 16 or 32
+// rows: they pay while the wide tiles leave most CUs without a block, not by
+// the rows of an expert alone. Times in us of whole layers, top-2 unless
+// noted, over 912 measured layers (1 to 4,096 tokens, 4 to 64 experts).
+// Gate/up (128-wide tiles: B blocks), wide / K-split: 16 tokens, 512 x 1368, 4
+// experts (B 44) 47 / 42; 400 tokens, 1024 x 4096, 4 experts (B 320, 200 rows)
+// 78 / 132; at B 97..128 and 33..64 rows K-split loses by 7-14%.
+// Down (256-wide tiles: B blocks), best wide / K-split 16x32 / 32x32 / 32x64:
+//   1024 x 4096, 8 experts: 16 tokens (B 32) 84 / 64 / 66 / 68
+//   4096 x 1536, 8 experts: 128 tokens (B 160, 32 rows) 112 / 145 / 130 / 120
+//   1024 x 4096, 4 experts: 400 tokens (B 40, 200 rows) 95 / 114 / 99 / 78
+//   1024 x 4096, 16 experts: 64 tokens (B 68, 8 rows) 120 / 102 / 105 / 100;
+//     1400 tokens (B 148, 175 rows) 235 / - / - / 301
+//   2048 x 1408, 8 experts: 512 tokens (B 128, 128 rows) 95 / - / - / 103
+//   1024 x 4096, 64 experts, top-8: 768 tokens (B 448, 96 rows) 520 / - / - / 773;
+//     8 tokens (B 256, 1 row) 288 / 267 / 276 / 265, but 2048 x 1408 219 / 229
+//     / 234 / 222: past 128 blocks only where K (ffn) is the longer side
+// Wide tiles: 128 columns while they fit one round of CUs (1024 tokens, 1024 x
+// 4096, 8 experts 201 -> 177); then 192 where they are more blocks than 256-wide
+// ones and still one round (2048 tokens ~216 blocks against 144: the down GEMM
+// 100.6 -> 94.3 us); else 256 (2048 tokens in 128-wide tiles, 288 blocks, 288
+// against 281).
+enum MoeTile { kMoeKw16x32, kMoeKw32x32, kMoeKw32x64, kMoeWide128, kMoeWide192, kMoeWide256 };
+struct MoeTiles {
+    MoeTile gate_up, down;  // gate_up: kMoeKw32x32 or kMoeWide128
+};
+static MoeTiles moe_tiles(int MK, int E, int d, int F) {
+    const int avg = MK / E;
+    const long long live = std::min(E, MK) + MK / kWideBM;
+    auto blocks = [&](int n, int bn) { return live * ((n + bn - 1) / bn); };
+    MoeTiles t;
+    const long long gu = blocks(F, kWideBNDual), down = blocks(d, kWideBNDown);
+    t.gate_up = (gu <= 96 && avg <= 64) || (gu <= 128 && avg <= 32) ? kMoeKw32x32 : kMoeWide128;
+    if (down <= 64 || (down <= 128 && avg <= 32) || (avg <= 8 && F >= 2 * d))
+        t.down = avg <= 8 && down <= 128 ? kMoeKw16x32 : avg <= 16 && down <= 128 ? kMoeKw32x32 : kMoeKw32x64;
+    else if (blocks(d, 128) <= 256) t.down = kMoeWide128;
+    else if (blocks(d, 192) <= 256 && blocks(d, 192) > down) t.down = kMoeWide192;
+    else t.down = kMoeWide256;
+    return t;
+}
+
+// The kernels' names (gorch_hip_kernel_choice).
+const char* moe_choice_name(int tokens, int dim, int ffn, int experts, int top_k, bool down) {
+    static const char* const kName[] = {"kw16x32", "kw32x32", "kw32x64", "wide128", "wide192", "wide256"};
+    const MoeTiles t = moe_tiles(tokens * top_k, experts, dim, ffn);
+    return kName[down ? t.down : t.gate_up];
+}
+
 }  // namespace gh
 
 using namespace gh;
@@ -975,20 +1023,9 @@ extern "C" int gorch_hip_moe_forward(void* stream, const gorch_hip_moe_weights* 
         hipLaunchKernelGGL(k_moe_gather_split<kMaxTopK>, dim3(gblocks), dim3(256), 0, s, x, ws.inv, xhi, xlo, M, K,
                            d);
     GH_TRY(check_launch("moe_gather"));
-    // At most this many row tiles are live: one per expert reached and one
-    // more per 128 rows. Few rows per expert: K split over the waves of small
-    // tiles (k_moe_kw), else the wide tiles. Down GEMM, whole layer in us (1024 x 4096, 8
-    // experts, top-2), wide / kw 16x32 / 32x32 / 32x64: 16 tokens (4 rows an
-    // expert) 103 / 64 / 66 / 68; 64 (16) 107 / 73 / 70 / 73; 128 (32) 110 /
-    // 84 / 76 / 72; 512 (128) 158 / 183 / 152 / 135; 1024 (256) 201 / - / 227
-    // / 217. With few column tiles the wide form stays short of CUs at any
-    // length (1000 tokens, 512 x 1368, 4 experts, 38 blocks: 74 / - / 67 / 61).
-    const int avg = MK / E;
-    const long long live = std::min(E, MK) + MK / tile_rows;
+    const MoeTiles tiles = moe_tiles(MK, E, d, F);
     auto chunks = [&](int bm) { return (unsigned)((std::min(M, tile_rows) + bm - 1) / bm); };
-    if (live * ((F + kWideBNDual - 1) / kWideBNDual) <= 128 && avg <= 64) {
-        // the wide form would run on half the CUs or fewer (16 tokens, 512 x
-        // 1368, 4 experts: 47 -> 42 us a layer)
+    if (tiles.gate_up == kMoeKw32x32) {
         hipLaunchKernelGGL((k_moe_kw<true, 32, 32, 4, 2>), dim3((F + 31) / 32, max_tiles, chunks(32)), dim3(256), 0, s,
                            xhi, xlo, w->wgate, w->wup, w->bgate, w->bup, nullptr, hhi, hlo, F, d, ws);
         GH_TRY(check_launch("moe_kw_gate_up"));
@@ -999,36 +1036,23 @@ extern "C" int gorch_hip_moe_forward(void* stream, const gorch_hip_moe_weights* 
     // the down GEMM unsplit over K (one slice of partials in yg)
     const int nsl = 1;
     const long long cslice = (long long)MK * d;
-    if (avg <= 192 || live * ((d + kWideBNDown - 1) / kWideBNDown) <= 64) {
-        if (avg <= 8)
-            hipLaunchKernelGGL((k_moe_kw<false, 16, 32, 8, 2>), dim3((d + 31) / 32, max_tiles, chunks(16)), dim3(512), 0, s,
-                               hhi, hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, ws);
-        else if (avg <= 16)
-            hipLaunchKernelGGL((k_moe_kw<false, 32, 32, 4, 3>), dim3((d + 31) / 32, max_tiles, chunks(32)), dim3(256), 0, s,
-                               hhi, hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, ws);
-        else
-            hipLaunchKernelGGL((k_moe_kw<false, 32, 64, 4, 2>), dim3((d + 63) / 64, max_tiles, chunks(32)), dim3(256), 0, s,
-                               hhi, hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, ws);
-        GH_TRY(check_launch("moe_kw_down"));
-    } else if (live * ((d + 127) / 128) <= 256) {
-        // 128-wide tiles while they still fit one round of CUs: 1024 tokens
-        // 201 -> 182 us a layer; past a round the 256-wide ones (2048 tokens,
-        // ~288 of these: 288 against 281)
-        GH_TRY((launch_moe_wide<false, 128>(s, dim3((d + 127) / 128, max_tiles, nsl), hhi, hlo, w->wdown, nullptr,
-                                            w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, cslice, ws)));
-    } else if (live * ((d + 191) / 192) <= 256 && (d + 191) / 192 > (d + 255) / 256) {
-        // in between, 192-wide tiles where they are more blocks and still one
-        // round (2048 tokens, 8 experts, 1024 columns: ~216 blocks against
-        // 144, the down GEMM 100.6 -> 94.3 us; whole layers of 1700 x 1024 x
-        // 4096, 1800 x 768 x 3072 and 2300 x 768 x 2048 248.7 -> 242.1, 167.0
-        // -> 160.4, 158.1 -> 152.9 us)
-        GH_TRY((launch_moe_wide<false, 192>(s, dim3((d + 191) / 192, max_tiles, nsl), hhi, hlo, w->wdown, nullptr,
-                                            w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, cslice, ws)));
-    } else {
-        GH_TRY((launch_moe_wide<false, kWideBNDown>(s, dim3((d + kWideBNDown - 1) / kWideBNDown, max_tiles, nsl), hhi,
-                                                    hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr,
-                                                    d, F, cslice, ws)));
+#define GH_DOWN_KW(BM, BN, G, NST)                                                                                  \
+    hipLaunchKernelGGL((k_moe_kw<false, BM, BN, G, NST>), dim3((d + BN - 1) / BN, max_tiles, chunks(BM)), dim3(64 * G), 0, s, \
+                       hhi, hlo, w->wdown, nullptr, w->bdown, nullptr, ws.yg, nullptr, nullptr, d, F, ws)
+#define GH_DOWN_WIDE(BN)                                                                                            \
+    GH_TRY((launch_moe_wide<false, BN>(s, dim3((d + BN - 1) / BN, max_tiles, nsl), hhi, hlo, w->wdown, nullptr, w->bdown, \
+                                       nullptr, ws.yg, nullptr, nullptr, d, F, cslice, ws)))
+    switch (tiles.down) {
+        case kMoeKw16x32: GH_DOWN_KW(16, 32, 8, 2); break;
+        case kMoeKw32x32: GH_DOWN_KW(32, 32, 4, 3); break;
+        case kMoeKw32x64: GH_DOWN_KW(32, 64, 4, 2); break;
+        case kMoeWide128: GH_DOWN_WIDE(128); break;
+        case kMoeWide192: GH_DOWN_WIDE(192); break;
+        default: GH_DOWN_WIDE(kWideBNDown); break;
     }
+#undef GH_DOWN_KW
+#undef GH_DOWN_WIDE
+    GH_TRY(check_launch("moe_down"));
     const int cblocks = (int)std::min<int64_t>(8192, ((int64_t)M * d / 4 + 255) / 256);
     if (K <= 2)
         hipLaunchKernelGGL(k_moe_combine<2>, dim3(cblocks), dim3(256), 0, s, ws.yg, ws.inv, ws.topi, out, M, K, d, nsl,

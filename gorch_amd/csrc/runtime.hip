@@ -491,6 +491,9 @@ const char* gorch_hip_kernel_choice(const char* op, const int* d, int n) {
         return gemm_pair_swiglu_ok(d[0], d[1], d[2]) ? "pair64x64" : gemm_choice_name(d[0], 2 * d[1], d[2], false);
     if (is("matmul", 6) && d[0] > 0 && d[1] > 0 && d[2] > 0 && d[3] > 0)
         return matmul_choice_name(d[0], d[1], d[2], d[3], d[4] != 0, d[5] != 0);
+    const bool moe_up = is("moe_gate_up", 5);
+    if ((moe_up || is("moe_down", 5)) && d[0] > 0 && d[1] > 0 && d[2] > 0 && d[3] > 0 && d[4] > 0)
+        return moe_choice_name(d[0], d[1], d[2], d[3], d[4], !moe_up);
     if (is("attention", 7) && d[0] > 0 && d[1] > 0 && d[3] > 0 && d[5] > 0 && (!d[4] || d[3] % d[4] == 0))
         return attn_choice_name(d[0], d[1], d[2], d[3], d[4], d[5], d[6]);
     return nullptr;

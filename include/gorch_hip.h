@@ -147,6 +147,8 @@ void gorch_hip_reset_dispatch_counts(void);
  *     above 16 rows ("pair...": in one kernel);
  *   "matmul" {M, N, K, batch, aBF16, bBF16}: the general product
  *     (gorch_hip_matmul_dt's route to the Linear aside);
+ *   "moe_gate_up", "moe_down" {tokens, dim, ffn, experts, top_k}: the tiles of
+ *     gorch_hip_moe_forward's expert GEMMs;
  *   "attention" {batch, new rows, cached rows, heads, KV heads (0: one per
  *     head), head_dim, max_seq}: a causal attention_cached call over 16-byte
  *     aligned buffers.

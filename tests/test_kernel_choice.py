@@ -130,3 +130,24 @@ MATMUL = [
 @pytest.mark.parametrize("dims,name", MATMUL, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v)
 def test_matmul_kernel(dims, name):
     assert hip.kernel_choice("matmul", *dims) == name
+
+
+# op, tokens, dim, ffn, experts, top-k
+MOE = [
+    # many experts fill the CUs with wide tiles however few rows each has: the
+    # K-split down tiles took 1.1 to 1.6 times as long a layer
+    (("moe_down", 1400, 1024, 4096, 16, 2), {"wide192", "wide256"}), (("moe_down", 768, 1024, 4096, 64, 8), {"wide256", "wide192"}),
+    (("moe_down", 512, 2048, 1408, 64, 8), {"wide256", "wide192"}), (("moe_down", 768, 2048, 1408, 8, 2), {"wide128", "wide192"}),
+    (("moe_down", 400, 2048, 1408, 8, 2), {"wide128"}), (("moe_gate_up", 128, 1024, 1408, 8, 2), {"kw32x32", "wide128"}),
+    (("moe_gate_up", 200, 2048, 1408, 8, 2), {"wide128"}),
+    # the right ones before
+    (("moe_down", 16, 1024, 4096, 8, 2), {"kw16x32"}), (("moe_down", 400, 1024, 4096, 4, 2), {"kw32x64"}),
+    (("moe_down", 64, 1024, 4096, 16, 2), {"kw32x32", "kw32x64", "kw16x32"}), (("moe_down", 2048, 1024, 4096, 8, 2), {"wide192"}),
+    (("moe_down", 1024, 1024, 4096, 8, 2), {"wide128"}), (("moe_gate_up", 16, 512, 1368, 4, 2), {"kw32x32"}),
+    (("moe_gate_up", 2048, 1024, 4096, 8, 2), {"wide128"}), (("moe_gate_up", 16, 1024, 4096, 8, 2), {"wide128"}),
+]
+
+
+@pytest.mark.parametrize("dims,names", MOE, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "")
+def test_moe_tiles(dims, names):
+    assert hip.kernel_choice(*dims) in names
