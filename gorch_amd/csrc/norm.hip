@@ -46,12 +46,13 @@ __global__ __launch_bounds__(256) void k_layernorm(const float* __restrict__ x, 
     }
 }
 
-// Rows of at most 1024 R floats (N % 4 == 0, 16-byte rows and gains): a block
-// per row holds it in registers, R float4 a thread, so the two f64 passes
-// (mean, then squared deviations) and the output cost one trip to memory
-// instead of three; the gains are requested with the row. Same statistics
-// and f32 operations as k_layernorm. Latency for few rows (64 x 768: 3.5 ->
-// 2.5 us in a graph), HBM for many (8192 x 1600: 33.8 -> 16.8 us, 6.3 TB/s).
+// Rows of at most 1024 R floats (N % 4 == 0, x and y 16-byte aligned; the
+// gains' buffer loads need 4 bytes only): a block per row holds it in
+// registers, R float4 a thread, so the two f64 passes (mean, then squared
+// deviations) and the output cost one trip to memory instead of three; the
+// gains are requested with the row. Same statistics and f32 operations as
+// k_layernorm. Latency for few rows (64 x 768: 3.5 -> 2.5 us in a graph),
+// HBM for many (8192 x 1600: 33.8 -> 16.8 us, 6.3 TB/s).
 template <int R>
 __global__ __launch_bounds__(256) void k_layernorm_rows(const float* __restrict__ x, const float* __restrict__ g,
                                                         const float* __restrict__ b, float* __restrict__ y, int N,
