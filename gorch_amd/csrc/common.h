@@ -569,9 +569,9 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 // 7.8 (36: 1 + tanh cancels there). x / (1 + exp(-2u)) on the same two
 // instructions has 4.7 (3.8) at 1. Linears with GELU against tanhf: 512 x 768 x
 // 3072 14.1 -> 13.0 us (64-row tiles); against that shorter form 8192 x 768 x
-// 3072 81.5 -> 85.1, 8192 x 1600 x 6400 305 -> 306 (256-row tiles). The GEMVs keep tanhf: it is not on their
-// path's bound, and the tile GEMV compiled with a form like this ran slower
-// (LM head of 16 rows 15.8 -> 16.8 us).
+// 3072 81.5 -> 85.1, 8192 x 1600 x 6400 307 -> 310 (256-row tiles). The GEMVs
+// keep tanhf: it is not on their path's bound, and the tile GEMV compiled with
+// a form like this ran slower (LM head of 16 rows 15.8 -> 16.8 us).
 __device__ __forceinline__ float gelu_gemm(float x) {
     const float ax = fabsf(x);
     const float c = __builtin_fmaf(x * x, -0.10294324f, -2.3022082f);  // -2 log2(e) u / x

@@ -487,7 +487,7 @@ const char* gorch_hip_kernel_choice(const char* op, const int* d, int n) {
     const auto is = [&](const char* name, int count) { return n == count && !strcmp(op, name); };
     if (is("linear", 4) && d[0] > 0 && d[1] > 0)
         return gemm_choice_name(d[0], d[1], d[2], (d[3] & GORCH_HIP_LINEAR_ACT_BF16) != 0);
-    if (is("gate_up", 3) && d[0] > 16 && d[1] > 0)
+    if (is("gate_up", 3) && d[0] > 16 && d[1] > 0 && d[1] < 1 << 30)
         return gemm_pair_swiglu_ok(d[0], d[1], d[2]) ? "pair64x64" : gemm_choice_name(d[0], 2 * d[1], d[2], false);
     if (is("matmul", 6) && d[0] > 0 && d[1] > 0 && d[2] > 0 && d[3] > 0)
         return matmul_choice_name(d[0], d[1], d[2], d[3], d[4] != 0, d[5] != 0);

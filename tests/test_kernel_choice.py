@@ -15,6 +15,7 @@ def test_unknown_names_and_sizes():
     assert hip.kernel_choice("no such op", 64, 64, 64, 0) is None
     assert hip.kernel_choice("linear", -1, 64, 64, 0) is None
     assert hip.kernel_choice("linear", 0, 64, 64, 0) is None
+    assert hip.kernel_choice("gate_up", 17, (1 << 31) - 1, 64) is None
 
 
 # rows, columns, K, flags: the fastest kernels
